@@ -9,7 +9,10 @@
 //
 // Row-split: a group of G lanes owns one row, each lane 4 adjacent columns
 // (float4), so a wave covers 64/G rows and one B row gather per nonzero is a
-// single coalesced G*16-byte access.  The row's (col, val) pairs are loaded
+// single coalesced G*16-byte access.  Widths that are not a multiple of 4 and
+// operands that are not 16-byte aligned take the same kernels: the float4
+// accesses only need 4-byte alignment, and the last lane of a row moves
+// back to columns N-4..N-1.  The row's (col, val) pairs are loaded
 // cooperatively by the group and broadcast by lane shuffles, U B-rows in
 // flight per group.  Stated accumulation order (bit-identical to the CPU loop
 // of oracle_spmm_csr):
@@ -68,14 +71,97 @@ __device__ __forceinline__ void register_row(LongCtl *ctl, LongRow *longs, int32
   for (int32_t q = 0; q < nseg; ++q) owner[base + q] = id;
 }
 
-__device__ __forceinline__ float4 scale4(float d, float4 v) {
+// The V adjacent columns of a dense row that one lane holds: a float4, or a
+// float for rows narrower than 4.  RG (ragged): the rows start on any multiple
+// of 4 bytes, which is all global_load_dwordx4 and the store need.  It is a
+// template argument so that aligned whole widths keep the compiler's 16-byte
+// accesses and hold no moved column: the scaled kernel then fits 80 registers,
+// 6 waves per SIMD (forward and backward of a 2.4 M-row power-law graph's
+// scaled product at N = 128: 8.15 ms, and 8.68 ms with 86 registers).
+template <int V> struct ColsOf {
+  typedef float4 T;
+  typedef float Mem __attribute__((ext_vector_type(4), aligned(4)));
+};
+template <> struct ColsOf<1> {
+  typedef float T;
+};
+
+template <int V, bool RG>
+__device__ __forceinline__ typename ColsOf<V>::T load_cols(const float *src) {
+  if constexpr (V == 1) {
+    return *src;
+  } else if constexpr (RG) {
+    const ColsOf<4>::Mem m = *reinterpret_cast<const ColsOf<4>::Mem *>(src);
+    return make_float4(m.x, m.y, m.z, m.w);
+  } else {
+    return *reinterpret_cast<const float4 *>(src);
+  }
+}
+
+template <bool RG> __device__ __forceinline__ void store_cols(float *dst, float4 v) {
+  if constexpr (RG) {
+    *reinterpret_cast<ColsOf<4>::Mem *>(dst) = ColsOf<4>::Mem{v.x, v.y, v.z, v.w};
+  } else {
+    *reinterpret_cast<float4 *>(dst) = v;
+  }
+}
+template <bool RG> __device__ __forceinline__ void store_cols(float *dst, float v) { *dst = v; }
+
+// Non-temporal; RG: without the first `skip` elements (another lane's).
+template <bool RG> __device__ __forceinline__ void store_nt(float *dst, float4 v, int skip) {
+  if (RG && skip != 0) {
+    if (skip <= 1) __builtin_nontemporal_store(v.y, dst + 1);
+    if (skip <= 2) __builtin_nontemporal_store(v.z, dst + 2);
+    __builtin_nontemporal_store(v.w, dst + 3);
+  } else if constexpr (RG) {
+    __builtin_nontemporal_store(ColsOf<4>::Mem{v.x, v.y, v.z, v.w},
+                                reinterpret_cast<ColsOf<4>::Mem *>(dst));
+  } else {
+    __builtin_nontemporal_store(v.x, dst + 0);
+    __builtin_nontemporal_store(v.y, dst + 1);
+    __builtin_nontemporal_store(v.z, dst + 2);
+    __builtin_nontemporal_store(v.w, dst + 3);
+  }
+}
+template <bool RG> __device__ __forceinline__ void store_nt(float *dst, float v, int) {
+  __builtin_nontemporal_store(v, dst);
+}
+
+__device__ __forceinline__ float4 scaled(float d, float4 v) {
   return make_float4(d * v.x, d * v.y, d * v.z, d * v.w);
 }
+__device__ __forceinline__ float scaled(float d, float v) { return d * v; }
+
+__device__ __forceinline__ float4 fma_cols(float v, float4 b, float4 acc) {
+  return make_float4(fmaf(v, b.x, acc.x), fmaf(v, b.y, acc.y), fmaf(v, b.z, acc.z),
+                     fmaf(v, b.w, acc.w));
+}
+__device__ __forceinline__ float fma_cols(float v, float b, float acc) { return fmaf(v, b, acc); }
+
+__device__ __forceinline__ float4 added(float4 a, float4 b) {
+  return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+}
+__device__ __forceinline__ float added(float a, float b) { return a + b; }
+
+template <int V> __device__ __forceinline__ typename ColsOf<V>::T zero_cols();
+template <> __device__ __forceinline__ float4 zero_cols<4>() {
+  return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+}
+template <> __device__ __forceinline__ float zero_cols<1>() { return 0.0f; }
 
 // The row scale applied to a finished row (rs null: none), rounded once per
 // element: the value an elementwise product of the result would hold.
-__device__ __forceinline__ float4 row_scaled(const float *__restrict__ rs, int64_t row, float4 v) {
-  return rs != nullptr ? scale4(rs[row], v) : v;
+template <typename T>
+__device__ __forceinline__ T row_scaled(const float *__restrict__ rs, int64_t row, T v) {
+  return rs != nullptr ? scaled(rs[row], v) : v;
+}
+
+// A lane's first column when its slice starts at `at` < N.  Ragged widths (RG:
+// N not a multiple of V): the last slice starts at N - V and repeats up to
+// V - 1 columns of the slice before it (the same values; stored by that one
+// only).
+template <int V, bool RG> __device__ __forceinline__ int32_t slice_col(int32_t at, int32_t N) {
+  return !RG || at + V <= N ? at : N - V;
 }
 
 // A[s, e) x B on the group's float4 column slice col0 (col_ok false: lanes
@@ -85,14 +171,13 @@ __device__ __forceinline__ float4 row_scaled(const float *__restrict__ rs, int64
 // multiplied by cs[p] (the scale of that nonzero's column, streamed beside
 // the values), cs[p] * B[col][j] rounded once: the value an elementwise
 // product of B by a column-scale vector would hold.
-template <int G, bool CS>
-__device__ __forceinline__ float4 group_dot(int32_t s, int32_t e, const int32_t *__restrict__ ind,
-                                            const float *__restrict__ val, int32_t N,
-                                            int32_t col0, bool col_ok,
-                                            const float *__restrict__ B, int gl, int gbase,
-                                            const float *__restrict__ cs) {
+template <int G, bool CS, int V, bool RG>
+__device__ __forceinline__ typename ColsOf<V>::T
+group_dot(int32_t s, int32_t e, const int32_t *__restrict__ ind, const float *__restrict__ val,
+          int32_t N, int32_t col0, bool col_ok, const float *__restrict__ B, int gl, int gbase,
+          const float *__restrict__ cs) {
   constexpr int U = kSpmmDepth;
-  float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  typename ColsOf<V>::T acc = zero_cols<V>();
   for (int32_t pb = s;; pb += G) {
     const int32_t rem = e - pb;
     if (ballot(rem > 0) == 0) break;
@@ -110,7 +195,7 @@ __device__ __forceinline__ float4 group_dot(int32_t s, int32_t e, const int32_t 
     for (int32_t t = 0; t < cmax; t += U) {
       int32_t c[U];
       float v[U], d[U];
-      float4 b[U];
+      typename ColsOf<V>::T b[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         c[u] = __shfl(my_c, gbase + ((t + u) & (G - 1)), kWave);
@@ -119,7 +204,7 @@ __device__ __forceinline__ float4 group_dot(int32_t s, int32_t e, const int32_t 
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (t + u < cnt && col_ok) {
-          b[u] = *reinterpret_cast<const float4 *>(B + static_cast<int64_t>(c[u]) * N + col0);
+          b[u] = load_cols<V, RG>(B + static_cast<int64_t>(c[u]) * N + col0);
         }
       }
       // Each lane loaded its own nonzero's column scale; it is shared out only
@@ -131,23 +216,13 @@ __device__ __forceinline__ float4 group_dot(int32_t s, int32_t e, const int32_t 
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (t + u < cnt && col_ok) {
-          if constexpr (CS) b[u] = scale4(d[u], b[u]);
-          acc.x = fmaf(v[u], b[u].x, acc.x);
-          acc.y = fmaf(v[u], b[u].y, acc.y);
-          acc.z = fmaf(v[u], b[u].z, acc.z);
-          acc.w = fmaf(v[u], b[u].w, acc.w);
+          if constexpr (CS) b[u] = scaled(d[u], b[u]);
+          acc = fma_cols(v[u], b[u], acc);
         }
       }
     }
   }
   return acc;
-}
-
-__device__ __forceinline__ void store_nt(float *dst, float4 v) {
-  __builtin_nontemporal_store(v.x, dst + 0);
-  __builtin_nontemporal_store(v.y, dst + 1);
-  __builtin_nontemporal_store(v.z, dst + 2);
-  __builtin_nontemporal_store(v.w, dst + 3);
 }
 
 // One pass over the rows, 64/G rows per wave, one wave per row set (no grid
@@ -156,7 +231,7 @@ __device__ __forceinline__ void store_nt(float *dst, float4 v) {
 // C is written with non-temporal stores: it is not read again by this launch
 // and would only evict B from the caches.  rs / cs (CS): the row scales and
 // the per-nonzero column scales of a scaled product (null rs: none).
-template <int G, bool CS>
+template <int G, bool CS, int V, bool RG>
 __global__ void __launch_bounds__(kSpmmBlock)
     spmm_rowsplit_v4(int32_t n, const int32_t *__restrict__ ptr,
                      const int32_t *__restrict__ ind,
@@ -195,10 +270,13 @@ __global__ void __launch_bounds__(kSpmmBlock)
     if (gl == 0) register_row(ctl, longs, owner, static_cast<int32_t>(row), e - s);
     s = e; // the segment launch computes this row
   }
-  for (int32_t col0 = gl * 4; col0 - gl * 4 < N; col0 += G * 4) {
-    const bool col_ok = col0 < N;
-    const float4 acc = group_dot<G, CS>(s, e, ind, val, N, col0, col_ok, B, gl, gbase, cs);
-    if (row_ok && col_ok && !is_long) store_nt(C + row * N + col0, row_scaled(rs, row, acc));
+  for (int32_t at = gl * V; at - gl * V < N; at += G * V) {
+    const bool col_ok = at < N;
+    const int32_t col0 = slice_col<V, RG>(at, N);
+    const auto acc = group_dot<G, CS, V, RG>(s, e, ind, val, N, col0, col_ok, B, gl, gbase, cs);
+    if (row_ok && col_ok && !is_long) {
+      store_nt<RG>(C + row * N + col0, row_scaled(rs, row, acc), RG ? at - col0 : 0);
+    }
   }
 }
 
@@ -209,7 +287,7 @@ __global__ void __launch_bounds__(kSpmmBlock)
 // fmaf chain in CSR order.  Row bounds come from one coalesced load of the
 // wave's 65 row pointers; rows longer than kLongRow are registered for the
 // segment launch as in spmm_rowsplit_v4.
-template <int G, bool CS>
+template <int G, bool CS, int V, bool RG>
 __global__ void __launch_bounds__(kSpmmBlock)
     spmm_rows_dyn(int32_t n, const int32_t *__restrict__ ptr, const int32_t *__restrict__ ind,
                   const float *__restrict__ val, int32_t N, const float *__restrict__ B,
@@ -231,14 +309,14 @@ __global__ void __launch_bounds__(kSpmmBlock)
   // Lane i holds ptr[r0 + i] (i <= nrows); ptr[r0 + 64] separately.
   const int32_t pl = ptr[r0 + (lane < nrows ? lane : nrows)];
   const int32_t p_last = ptr[r0 + nrows];
-  const int col0 = gl * 4;
-  const bool col_ok = col0 < N;
+  const bool col_ok = gl * V < N;
+  const int32_t col0 = slice_col<V, RG>(gl * V, N);
 
   int32_t row = sub < nrows ? sub : -1; // local row of this group, -1 idle
   int32_t next = RPW;                   // wave-uniform: next unclaimed local row
   int32_t p = 0, e = 0;
   bool is_long = false;
-  float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  typename ColsOf<V>::T acc = zero_cols<V>();
   // A claimed row longer than kLongRow goes to the segment launch and counts
   // as finished at once.
   auto take_long = [&]() {
@@ -264,7 +342,8 @@ __global__ void __launch_bounds__(kSpmmBlock)
     while (true) {
       const bool fin = row >= 0 && p >= e;
       if (fin && !is_long && col_ok) {
-        store_nt(C + (r0 + row) * N + col0, row_scaled(rs, r0 + row, acc));
+        store_nt<RG>(C + (r0 + row) * N + col0, row_scaled(rs, r0 + row, acc),
+                 RG ? gl * V - col0 : 0);
       }
       const uint64_t fmask = ballot(fin && gl == 0);
       if (fmask == 0) break;
@@ -280,7 +359,7 @@ __global__ void __launch_bounds__(kSpmmBlock)
         p = row >= 0 ? a : 0;
         e = row >= 0 ? b : 0;
         is_long = false;
-        acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        acc = zero_cols<V>();
         take_long();
       }
       next += __popcll(fmask);
@@ -300,7 +379,7 @@ __global__ void __launch_bounds__(kSpmmBlock)
     for (int32_t t = 0; t < cmax; t += U) {
       int32_t c[U];
       float v[U], d[U];
-      float4 bv[U];
+      typename ColsOf<V>::T bv[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         c[u] = __shfl(my_c, gbase + ((t + u) & (G - 1)), kWave);
@@ -309,7 +388,7 @@ __global__ void __launch_bounds__(kSpmmBlock)
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (t + u < cnt && col_ok) {
-          bv[u] = *reinterpret_cast<const float4 *>(B + static_cast<int64_t>(c[u]) * N + col0);
+          bv[u] = load_cols<V, RG>(B + static_cast<int64_t>(c[u]) * N + col0);
         }
       }
       if constexpr (CS) {
@@ -319,11 +398,8 @@ __global__ void __launch_bounds__(kSpmmBlock)
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (t + u < cnt && col_ok) {
-          if constexpr (CS) bv[u] = scale4(d[u], bv[u]);
-          acc.x = fmaf(v[u], bv[u].x, acc.x);
-          acc.y = fmaf(v[u], bv[u].y, acc.y);
-          acc.z = fmaf(v[u], bv[u].z, acc.z);
-          acc.w = fmaf(v[u], bv[u].w, acc.w);
+          if constexpr (CS) bv[u] = scaled(d[u], bv[u]);
+          acc = fma_cols(v[u], bv[u], acc);
         }
       }
     }
@@ -337,7 +413,7 @@ __global__ void __launch_bounds__(kSpmmBlock)
 // next launch: handing them over inside this one would need a device-scope
 // release/acquire per unit, which on MI355X writes back and invalidates the
 // XCD's L2 and so evicts every other wave's B rows.
-template <int G, bool CS>
+template <int G, bool CS, int V, bool RG>
 __global__ void __launch_bounds__(kSpmmBlock)
     spmm_long_segments(const int32_t *__restrict__ ptr, const int32_t *__restrict__ ind,
                        const float *__restrict__ val, int32_t N,
@@ -360,17 +436,20 @@ __global__ void __launch_bounds__(kSpmmBlock)
       s = rs + static_cast<int32_t>(u - lr.base) * kSegLen;
       e = s + kSegLen < re ? s + kSegLen : re;
     }
-    for (int32_t col0 = gl * 4; col0 - gl * 4 < N; col0 += G * 4) {
-      const bool col_ok = col0 < N;
-      const float4 acc = group_dot<G, CS>(s, e, ind, val, N, col0, col_ok, B, gl, gbase, cs);
-      if (ok && col_ok) *reinterpret_cast<float4 *>(part + u * N + col0) = acc;
+    for (int32_t at = gl * V; at - gl * V < N; at += G * V) {
+      const bool col_ok = at < N;
+      const int32_t col0 = slice_col<V, RG>(at, N);
+      const auto acc = group_dot<G, CS, V, RG>(s, e, ind, val, N, col0, col_ok, B, gl, gbase, cs);
+      // A moved-back slice rewrites its neighbour's last columns with the
+      // same values.
+      if (ok && col_ok) store_cols<RG>(part + u * N + col0, acc);
     }
   }
 }
 
 // C[row] = ((P_0 + P_1) + P_2) + ... for each long row, one row group per row,
 // eight partial rows in flight; then the row scale (rs null: none).
-template <int G>
+template <int G, int V, bool RG>
 __global__ void __launch_bounds__(kSpmmBlock)
     spmm_long_fixup(int32_t N, float *__restrict__ C, const LongCtl *__restrict__ ctl,
                     const LongRow *__restrict__ longs, const float *__restrict__ part,
@@ -384,37 +463,30 @@ __global__ void __launch_bounds__(kSpmmBlock)
   for (int64_t t = wave0 * kRowsPerWave + sub; t < rows; t += nwaves * kRowsPerWave) {
     const LongRow lr = longs[t];
     const float *p0 = part + static_cast<int64_t>(lr.base) * N;
-    for (int32_t col0 = gl * 4; col0 < N; col0 += G * 4) {
-      float4 sum = *reinterpret_cast<const float4 *>(p0 + col0);
+    for (int32_t at = gl * V; at < N; at += G * V) {
+      const int32_t col0 = slice_col<V, RG>(at, N);
+      typename ColsOf<V>::T sum = load_cols<V, RG>(p0 + col0);
       int32_t q = 1;
       for (; q + 8 <= lr.nseg; q += 8) {
-        float4 v[8];
+        typename ColsOf<V>::T v[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-          v[i] = *reinterpret_cast<const float4 *>(p0 + static_cast<int64_t>(q + i) * N + col0);
+        for (int i = 0; i < 8; ++i) v[i] = load_cols<V, RG>(p0 + static_cast<int64_t>(q + i) * N + col0);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          sum.x = sum.x + v[i].x;
-          sum.y = sum.y + v[i].y;
-          sum.z = sum.z + v[i].z;
-          sum.w = sum.w + v[i].w;
-        }
+        for (int i = 0; i < 8; ++i) sum = added(sum, v[i]);
       }
       for (; q < lr.nseg; ++q) {
-        const float4 v = *reinterpret_cast<const float4 *>(p0 + static_cast<int64_t>(q) * N + col0);
-        sum.x = sum.x + v.x;
-        sum.y = sum.y + v.y;
-        sum.z = sum.z + v.z;
-        sum.w = sum.w + v.w;
+        sum = added(sum, load_cols<V, RG>(p0 + static_cast<int64_t>(q) * N + col0));
       }
-      store_nt(C + static_cast<int64_t>(lr.row) * N + col0, row_scaled(rs, lr.row, sum));
+      store_nt<RG>(C + static_cast<int64_t>(lr.row) * N + col0, row_scaled(rs, lr.row, sum),
+               RG ? at - col0 : 0);
     }
   }
 }
 
-// Scalar fallback for widths that are not a multiple of 4 (or unaligned
-// operands): one wave per row, lanes over columns, same stated order (long
-// rows as segment chains added left to right).
+// One wave per row, lanes over columns, one gather in flight, same stated
+// order (long rows as segment chains added left to right) with no scratch: the
+// no-allocation entry's way for widths that are not a multiple of 4 whose long
+// rows need more scratch than it has.
 __global__ void __launch_bounds__(kSpmmBlock)
     spmm_rowsplit_scalar(int32_t n, const int32_t *__restrict__ ptr,
                          const int32_t *__restrict__ ind,
@@ -505,7 +577,7 @@ __global__ void __launch_bounds__(kSpmmBlock)
 // a window of G row pointers held in the group's lanes; empty rows are
 // skipped (the prepare launch zeroes them).  N > 4G is covered by repeating
 // the walk per column slice.
-template <int G>
+template <int G, bool RG>
 __global__ void __launch_bounds__(kSpmmBlock)
     spmm_merge_v4(int32_t n, int32_t nnz, const int32_t *__restrict__ ptr,
                   const int32_t *__restrict__ ind, const float *__restrict__ val, int32_t N,
@@ -525,8 +597,9 @@ __global__ void __launch_bounds__(kSpmmBlock)
   // First row of the span: the row holding nonzero p0 (from the prepare launch).
   const int32_t first = has ? start_row[grp] : -1;
   for (int32_t cb = 0; cb < N; cb += 4 * G) {
-    const int32_t col0 = cb + gl * 4;
-    const bool col_ok = col0 < N;
+    const int32_t at = cb + gl * 4;
+    const bool col_ok = at < N;
+    const int32_t col0 = slice_col<4, RG>(at, N);
     int32_t row = first;
     int32_t wbase = first >= 0 ? first : 0;
     int32_t win = ptr[wbase + 1 + gl < n ? wbase + 1 + gl : n]; // ptr[wbase + 1 + gl]
@@ -535,7 +608,7 @@ __global__ void __launch_bounds__(kSpmmBlock)
     int32_t re = row >= 0 ? w0 : 0;
     int32_t p = row >= 0 ? (rs > p0 ? rs : p0) : 0;
     int32_t e = row >= 0 ? (re < p1 ? re : p1) : 0;
-    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float4 acc = zero_cols<4>();
     while (true) {
       // Retire finished pieces and move each such group to its span's next
       // row, until every group has work or is done.
@@ -544,11 +617,11 @@ __global__ void __launch_bounds__(kSpmmBlock)
         if (fin && col_ok) {
           float *dst = C + static_cast<int64_t>(row) * N + col0;
           if (rs >= p0 && re <= p1) {
-            store_nt(dst, acc);
+            store_nt<RG>(dst, acc, RG ? at - col0 : 0);
           } else {
-            atomicAdd(dst + 0, acc.x);
-            atomicAdd(dst + 1, acc.y);
-            atomicAdd(dst + 2, acc.z);
+            if (!RG || col0 >= at) atomicAdd(dst + 0, acc.x);
+            if (!RG || col0 + 1 >= at) atomicAdd(dst + 1, acc.y);
+            if (!RG || col0 + 2 >= at) atomicAdd(dst + 2, acc.z);
             atomicAdd(dst + 3, acc.w);
           }
         }
@@ -586,7 +659,7 @@ __global__ void __launch_bounds__(kSpmmBlock)
             row = next;
             p = rs;
             e = re < p1 ? re : p1;
-            acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            acc = zero_cols<4>();
           } else {
             row = -1;
           }
@@ -615,17 +688,12 @@ __global__ void __launch_bounds__(kSpmmBlock)
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           if (t + u < cnt && col_ok) {
-            bv[u] = *reinterpret_cast<const float4 *>(B + static_cast<int64_t>(c[u]) * N + col0);
+            bv[u] = load_cols<4, RG>(B + static_cast<int64_t>(c[u]) * N + col0);
           }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          if (t + u < cnt && col_ok) {
-            acc.x = fmaf(v[u], bv[u].x, acc.x);
-            acc.y = fmaf(v[u], bv[u].y, acc.y);
-            acc.z = fmaf(v[u], bv[u].z, acc.z);
-            acc.w = fmaf(v[u], bv[u].w, acc.w);
-          }
+          if (t + u < cnt && col_ok) acc = fma_cols(v[u], bv[u], acc);
         }
       }
       if (row >= 0) p += cnt;
@@ -695,6 +763,12 @@ struct SpmmScale {
   const float *col = nullptr;
 };
 
+// Whether the dense rows are not all whole, aligned float4s.
+bool is_ragged(int32_t N, const float *B, const float *C) {
+  return N % 4 != 0 || reinterpret_cast<uintptr_t>(B) % 16 != 0 ||
+         reinterpret_cast<uintptr_t>(C) % 16 != 0;
+}
+
 struct SpmmLongWs {
   LongCtl *ctl;
   LongRow *longs;
@@ -714,7 +788,7 @@ SpmmLongWs take_long_ws(Context &ctx, int32_t nnz, int32_t N) {
   return w;
 }
 
-template <int G, bool CS>
+template <int G, bool CS, int V, bool RG>
 void launch_rowsplit_gs(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr,
                         const int32_t *ind, const float *val, int32_t N, const float *B,
                         float *C, const SpmmLongWs &w, int64_t seg_cap, int64_t long_cap,
@@ -730,14 +804,14 @@ void launch_rowsplit_gs(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr
   // wider rows the fixed assignment keeps more waves in flight.  With a tile
   // list only the listed tiles' rows are computed.
   const int64_t waves = tiles == nullptr ? ceil_div64(n, rpw) : ntiles * (kTileRows / rpw);
-  if (G <= 8 && N <= 4 * G) {
+  if (G <= 8 && N <= V * G) {
     const int64_t dyn_waves = tiles == nullptr ? ceil_div64(n, kWave) : ntiles;
     const int64_t blocks = ceil_div64(dyn_waves, kSpmmWaves);
-    spmm_rows_dyn<G, CS><<<dim3(static_cast<unsigned>(blocks)), kSpmmBlock, 0, ctx.stream>>>(
+    spmm_rows_dyn<G, CS, V, RG><<<dim3(static_cast<unsigned>(blocks)), kSpmmBlock, 0, ctx.stream>>>(
         n, ptr, ind, val, N, B, C, w.ctl, w.longs, w.owner, tiles, ntiles, rs, cs);
   } else {
     const int64_t blocks = ceil_div64(waves, kSpmmWaves);
-    spmm_rowsplit_v4<G, CS><<<dim3(static_cast<unsigned>(blocks)), kSpmmBlock, 0,
+    spmm_rowsplit_v4<G, CS, V, RG><<<dim3(static_cast<unsigned>(blocks)), kSpmmBlock, 0,
                               ctx.stream>>>(n, ptr, ind, val, N, B, C, w.ctl, w.longs,
                                             w.owner, tiles, ntiles, rs, cs);
   }
@@ -745,12 +819,26 @@ void launch_rowsplit_gs(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr
   if (!long_rows) return;
   // Persistent grid over the registered segment units (none: exits at once).
   const int g = ctx.grid_for(ceil_div64(seg_cap, rpw * kSpmmWaves), kSpmmBlock, 2);
-  spmm_long_segments<G, CS><<<g, kSpmmBlock, 0, ctx.stream>>>(ptr, ind, val, N, B, w.ctl,
+  spmm_long_segments<G, CS, V, RG><<<g, kSpmmBlock, 0, ctx.stream>>>(ptr, ind, val, N, B, w.ctl,
                                                                 w.longs, w.owner, w.part, cs);
   SP_LAUNCH_CHECK();
   const int gf = ctx.grid_for(ceil_div64(long_cap, rpw * kSpmmWaves), kSpmmBlock, 2);
-  spmm_long_fixup<G><<<gf, kSpmmBlock, 0, ctx.stream>>>(N, C, w.ctl, w.longs, w.part, rs);
+  spmm_long_fixup<G, V, RG><<<gf, kSpmmBlock, 0, ctx.stream>>>(N, C, w.ctl, w.longs, w.part, rs);
   SP_LAUNCH_CHECK();
+}
+
+template <int G, int V, bool RG>
+void launch_rowsplit_gr(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr,
+                        const int32_t *ind, const float *val, int32_t N, const float *B,
+                        float *C, const SpmmLongWs &w, int64_t seg_cap, int64_t long_cap,
+                        const int32_t *tiles, int64_t ntiles, const SpmmScale &sc) {
+  if (sc.col != nullptr) {
+    launch_rowsplit_gs<G, true, V, RG>(ctx, n, nnz, ptr, ind, val, N, B, C, w, seg_cap,
+                                       long_cap, tiles, ntiles, sc.row, sc.col);
+  } else {
+    launch_rowsplit_gs<G, false, V, RG>(ctx, n, nnz, ptr, ind, val, N, B, C, w, seg_cap,
+                                        long_cap, tiles, ntiles, sc.row, nullptr);
+  }
 }
 
 template <int G>
@@ -758,12 +846,12 @@ void launch_rowsplit_g(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr,
                        const int32_t *ind, const float *val, int32_t N, const float *B,
                        float *C, const SpmmLongWs &w, int64_t seg_cap, int64_t long_cap,
                        const int32_t *tiles, int64_t ntiles, const SpmmScale &sc) {
-  if (sc.col != nullptr) {
-    launch_rowsplit_gs<G, true>(ctx, n, nnz, ptr, ind, val, N, B, C, w, seg_cap, long_cap,
-                                tiles, ntiles, sc.row, sc.col);
+  if (is_ragged(N, B, C)) {
+    launch_rowsplit_gr<G, 4, true>(ctx, n, nnz, ptr, ind, val, N, B, C, w, seg_cap, long_cap,
+                                   tiles, ntiles, sc);
   } else {
-    launch_rowsplit_gs<G, false>(ctx, n, nnz, ptr, ind, val, N, B, C, w, seg_cap, long_cap,
-                                 tiles, ntiles, sc.row, nullptr);
+    launch_rowsplit_gr<G, 4, false>(ctx, n, nnz, ptr, ind, val, N, B, C, w, seg_cap, long_cap,
+                                    tiles, ntiles, sc);
   }
 }
 
@@ -785,17 +873,18 @@ void spmm_rowsplit(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr,
                    const SpmmScale &sc = SpmmScale{}) {
   if (seg_cap < 0) seg_cap = max_segments(nnz);
   if (long_cap < 0) long_cap = max_long_rows(nnz);
-  bool aligned = (N % 4 == 0) && (reinterpret_cast<uintptr_t>(B) % 16 == 0) &&
-                 (reinterpret_cast<uintptr_t>(C) % 16 == 0);
-  if (!aligned) {
-    SP_EXPECT(tiles == nullptr, "internal: tile lists need aligned float4 operands");
-    int g = ctx.grid_for(ceil_div64(n, kSpmmBlock / kWave), kSpmmBlock, 8);
-    spmm_rowsplit_scalar<<<g, kSpmmBlock, 0, ctx.stream>>>(n, ptr, ind, val, N, B, C, sc.row,
-                                                           sc.col);
-    SP_LAUNCH_CHECK();
+  // Every width and alignment takes the row groups, long rows in segments.
+  // The one-wave-per-row kernel that ragged widths took before has one gather
+  // in flight and walks a long row alone: N = 47 on a power-law graph of
+  // 300,000 rows, 7.8 M nonzeros and an 88,909-nonzero hub, 27.1 -> 0.34 ms.
+  // Rows narrower than 4: a lane per column, 8 lanes per row (each loads its
+  // share of the row's nonzeros).
+  if (N < 4) {
+    launch_rowsplit_gr<8, 1, false>(ctx, n, nnz, ptr, ind, val, N, B, C, w, seg_cap, long_cap, tiles,
+                            ntiles, sc);
     return;
   }
-  int32_t q = N / 4; // float4 columns
+  const int32_t q = (N + 3) / 4; // float4 column slices
   if (q <= 1) {
     launch_rowsplit_g<1>(ctx, n, nnz, ptr, ind, val, N, B, C, w, seg_cap, long_cap,
                           tiles, ntiles, sc);
@@ -850,18 +939,21 @@ void launch_merge_g(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr,
   SP_LAUNCH_CHECK();
   if (nnz == 0) return;
   const int64_t blocks = ceil_div64(spans, gpw * kSpmmWaves);
-  spmm_merge_v4<G><<<dim3(static_cast<unsigned>(blocks)), kSpmmBlock, 0, ctx.stream>>>(
-      n, nnz, ptr, ind, val, N, B, C, span, start_row);
+  if (is_ragged(N, B, C)) {
+    spmm_merge_v4<G, true><<<dim3(static_cast<unsigned>(blocks)), kSpmmBlock, 0, ctx.stream>>>(
+        n, nnz, ptr, ind, val, N, B, C, span, start_row);
+  } else {
+    spmm_merge_v4<G, false><<<dim3(static_cast<unsigned>(blocks)), kSpmmBlock, 0, ctx.stream>>>(
+        n, nnz, ptr, ind, val, N, B, C, span, start_row);
+  }
   SP_LAUNCH_CHECK();
 }
 
 void spmm_merge(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr,
                 const int32_t *ind, const float *val, int32_t N, const float *B,
                 float *C) {
-  const bool aligned = (N % 4 == 0) && (reinterpret_cast<uintptr_t>(B) % 16 == 0) &&
-                       (reinterpret_cast<uintptr_t>(C) % 16 == 0);
-  if (aligned) {
-    const int32_t q = N / 4; // float4 columns
+  if (N >= 4) {
+    const int32_t q = (N + 3) / 4; // float4 column slices
     if (q <= 1) {
       launch_merge_g<1>(ctx, n, nnz, ptr, ind, val, N, B, C);
     } else if (q <= 2) {
@@ -879,8 +971,7 @@ void spmm_merge(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr,
     }
     return;
   }
-  // Widths that are not a multiple of 4 (or unaligned operands): one wave per
-  // span, lanes over columns.
+  // Widths below 4: one wave per span, lanes over columns.
   int64_t slots = static_cast<int64_t>(ctx.num_cus) * (ctx.max_threads_per_cu / kWave) * 2;
   int64_t span64 = ceil_div64(nnz > 0 ? nnz : 1, slots);
   if (span64 < 32) span64 = 32;
@@ -987,17 +1078,6 @@ int32_t sporder_spmm_csr_noalloc(sporder_context_t h, int32_t n, int32_t nnz,
   Context &ctx = h->impl;
   char *base = static_cast<char *>(noalloc_scratch(ctx.device));
   std::lock_guard<std::mutex> call_lock(noalloc_call_mu[ctx.device]);
-  const bool aligned = (cols % 4 == 0) && (reinterpret_cast<uintptr_t>(d_b) % 16 == 0) &&
-                       (reinterpret_cast<uintptr_t>(d_c) % 16 == 0);
-  if (!aligned) {
-    // One wave per row in the stated order: no scratch.
-    int g = ctx.grid_for(ceil_div64(n, kSpmmBlock / kWave), kSpmmBlock, 8);
-    spmm_rowsplit_scalar<<<g, kSpmmBlock, 0, ctx.stream>>>(n, d_ptr, d_ind, d_val, cols, d_b,
-                                                           d_c);
-    SP_LAUNCH_CHECK();
-    ctx.sync();
-    return 0;
-  }
   // Exact need: count the long rows and their segments first.
   LongCtl *ctl = reinterpret_cast<LongCtl *>(base);
   fill_u32(ctx, ctl, sizeof(LongCtl) / 4, 0u);
@@ -1011,7 +1091,17 @@ int32_t sporder_spmm_csr_noalloc(sporder_context_t h, int32_t n, int32_t nnz,
   const size_t need = ws_bytes<LongCtl>(1) + ws_bytes<LongRow>(static_cast<size_t>(long_rows)) +
                       ws_bytes<int32_t>(static_cast<size_t>(segments)) +
                       ws_bytes<float>(static_cast<size_t>(segments) * cols);
-  if (need > kNoAllocBytes) return SPORDER_SPMM_NOALLOC_TOO_LARGE;
+  if (need > kNoAllocBytes) {
+    // A width of whole 16-byte slices on aligned operands is refused; any
+    // other takes the kernel that needs no scratch.
+    if (!is_ragged(cols, d_b, d_c)) return SPORDER_SPMM_NOALLOC_TOO_LARGE;
+    const int g = ctx.grid_for(ceil_div64(n, kSpmmBlock / kWave), kSpmmBlock, 8);
+    spmm_rowsplit_scalar<<<g, kSpmmBlock, 0, ctx.stream>>>(n, d_ptr, d_ind, d_val, cols, d_b,
+                                                           d_c);
+    SP_LAUNCH_CHECK();
+    ctx.sync();
+    return 0;
+  }
   SpmmLongWs w;
   size_t off = ws_bytes<LongCtl>(1);
   w.ctl = ctl;

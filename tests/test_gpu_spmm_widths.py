@@ -1,0 +1,76 @@
+"""The SpMM at widths that are not a multiple of 4 and on operands that start
+4, 8 or 12 bytes past a 16-byte boundary, bit for bit against the oracle, with
+guard words around the result: the last lane of a row moves back to columns
+N-4..N-1, rows narrower than 4 take a lane per column."""
+
+import numpy as np
+import pytest
+
+import oracle
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+N_ROWS = 1111
+
+
+@pytest.fixture(scope="module")
+def matrix():
+    """Rows of 0..80 nonzeros, and five around and past the 512-nonzero
+    segments (511, 512, 513, 1025, 1100)."""
+    rng = np.random.default_rng(21)
+    lens = rng.integers(0, 81, N_ROWS)
+    lens[[5, 64, 300, 777, N_ROWS - 1]] = [511, 512, 513, 1025, 1100]
+    lens[[0, 63, 128]] = 0
+    ind = np.concatenate([np.sort(rng.choice(N_ROWS, k, replace=False)) for k in lens])
+    ptr = np.concatenate([[0], np.cumsum(lens)])
+    val = rng.uniform(-1, 1, ind.size).astype(np.float32)
+    return ptr.astype(np.int32), ind.astype(np.int32), val
+
+
+def shifted(a, words):
+    """(buffer, view): a copy of `a` on the GPU that starts `words` floats
+    after an aligned start, 16 words of -7 on both sides."""
+    buf = torch.full((a.size + 32 + words,), -7.0, device=DEV)
+    view = buf[16 + words:16 + words + a.size].view(a.shape)
+    view.copy_(torch.from_numpy(a))
+    return buf, view
+
+
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 7, 13, 16, 17, 31, 33, 47, 64, 67, 127, 130, 259])
+@pytest.mark.parametrize("words", [0, 1, 2, 3])
+def test_spmm_widths_and_alignments(matrix, N, words):
+    from chunkedgreedy_amd import sporder
+
+    ptr, ind, val = matrix
+    rng = np.random.default_rng(N)
+    Bh = rng.standard_normal((N_ROWS, N)).astype(np.float32)
+    rs, cs = (rng.uniform(0.05, 2.0, N_ROWS).astype(np.float32) for _ in range(2))
+    want = oracle.spmm_csr(ptr, ind, val, Bh)
+    p, i, v = (torch.from_numpy(x).to(DEV) for x in matrix)
+    _, B = shifted(Bh, words)
+    buf, out = shifted(np.zeros_like(Bh), words)
+    plan = sporder.spmm_plan(p, i)
+
+    def check(what, ref):
+        got = out.cpu().numpy()
+        assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), what
+        assert torch.all(buf[:16 + words] == -7.0) and torch.all(buf[-16:] == -7.0), what
+        out.zero_()
+
+    print(f"[spmm_widths] N={N} words={words}", flush=True)
+    sporder.spmm_csr(p, i, v, B, out=out)
+    check("row_split", want)
+    sporder.spmm_csr(p, i, v, B, out=out, plan=plan)
+    check("plan", want)
+    sporder.spmm_csr_noalloc(p, i, v, B, out=out)
+    check("noalloc", want)
+    sporder.spmm_csr_scaled(p, i, v, B, row_scale=torch.from_numpy(rs).to(DEV),
+                            col_scale=torch.from_numpy(cs).to(DEV), out=out)
+    check("scaled", rs[:, None] * oracle.spmm_csr(ptr, ind, val, cs[:, None] * Bh))
+    sporder.spmm_csr(p, i, v, B, out=out, algo="merge_path")
+    scale = np.abs(want).max()
+    # A cut row adds its pieces in any order: rows of up to 1100 terms.
+    assert np.abs(out.cpu().numpy() - want).max() <= 1e-5 * scale
+    assert torch.all(buf[:16 + words] == -7.0) and torch.all(buf[-16:] == -7.0)
