@@ -24,10 +24,15 @@
 //      serial walk.
 //   4. sketch (one wave per row): walks the row's runs 64 nonzeros at a time
 //      with four blocks of runs in flight and item batches loaded one batch
-//      ahead, feeding the wave64 space-saving sketch (sketch.hpp).  An item's
+//      ahead, counting them in LDS while the row needs no eviction
+//      (row_count.hpp) and feeding the wave64 space-saving sketch (sketch.hpp)
+//      otherwise.  Finite-element matrix of 192,000 rows of 77 nonzeros (2,200
+//      items a row, capacity 320): the sketch 13.0 -> 2.6 ms; global sketch of
+//      a 2^18-point geometric graph: 3.34 -> 2.33 ms.  An item's
 //      run is found by marking run starts in LDS and a DPP running maximum.
 // The stream, and therefore the table, is the reference's.
 #include "common.hpp"
+#include "row_count.hpp"
 #include "sketch.hpp"
 
 namespace sporder_hip {
@@ -43,6 +48,7 @@ constexpr int kOvfBlock = 256;
 constexpr int kOvfWaves = kOvfBlock / kWave;
 constexpr int kMirrorBlock = 256;
 constexpr int kMirrorRowCap = 64; // longer rows: the whole wave (ovf_mirror_kernel)
+constexpr int kClaimRows = 16;   // most rows of one claim (ovf_sketch_kernel)
 constexpr int kSample = 16;      // run-search sample stride (one 64-byte line)
 
 __device__ __forceinline__ int64_t list_len(const int32_t *list, const int32_t *list_count,
@@ -208,21 +214,59 @@ __device__ __forceinline__ int32_t item_index(RunLookup *lk, int32_t len, int32_
   return f < total ? t : 0;
 }
 
-template <int CELLS>
-__device__ __forceinline__ void feed_batch(WaveSketch<CELLS> &store, int2 pr, int32_t f0,
-                                           int32_t total, int32_t row, int32_t deg,
-                                           int lane) {
-  const bool item = f0 + lane < total && pr.x != row;
-  const float alpha = 2.0f / static_cast<float>(deg + pr.y);
-  store.feed(ballot(item), pr.x, alpha);
-}
+// One row's stream: counted 64 items at a time (row_count.hpp) while it needs
+// no eviction, item by item in the sketch afterwards.
+template <int CELLS, bool WIDE> struct RowStream {
+  RowCounter<CELLS, row_table_entries(32 * CELLS), WIDE> counter;
+  WaveSketch<CELLS> store;
+  bool counting, opening; // wave-uniform; opening: no batch taken yet
+  const int32_t *row_ptr;
+  int32_t row, deg;
+  int32_t base; // candidates are counted as row - base
+
+  __device__ __forceinline__ void begin(int32_t r, int32_t d) {
+    row = r;
+    deg = d;
+    counting = true;
+    opening = true;
+  }
+  __device__ __forceinline__ int32_t size_of(int32_t s) const {
+    return row_ptr[s + 1] - row_ptr[s];
+  }
+  __device__ __forceinline__ void feed_batch(int2 pr, int32_t f0, int32_t total, int lane) {
+    const uint64_t items = ballot(f0 + lane < total && pr.x != row);
+    if (counting && opening) {
+      opening = false;
+      if (counter.add(items, static_cast<uint32_t>(pr.x - base)) &&
+          !counter.will_evict(total)) {
+        return;
+      }
+      // Evictions at once or ahead: this batch again, item by item.
+      counter.empty();
+      store.clear();
+      counting = false;
+    } else if (counting) {
+      if (counter.add(items, static_cast<uint32_t>(pr.x - base))) return;
+      counter.to_sketch(store, base, deg, [this](int32_t s) { return size_of(s); });
+      counting = false;
+    }
+    store.feed(items, pr.x, 2.0f / static_cast<float>(deg + pr.y));
+  }
+  __device__ __forceinline__ void finish(int32_t k, uint64_t *out) {
+    if (counting) {
+      counter.emit(store, k, out, base, deg, [this](int32_t s) { return size_of(s); });
+    } else {
+      store.select_top_k(k, out);
+    }
+  }
+};
 
 // One block of 64 runs through the sketch, item batches two at a time with
 // the second batch's load in flight while the first is applied.
-template <int CELLS>
-__device__ __forceinline__ void feed_block(WaveSketch<CELLS> &store, RunLookup *lk,
+template <typename Stream>
+__device__ __forceinline__ void feed_block(Stream &st, RunLookup *lk,
                                            const int2 *__restrict__ pairs, int2 run,
-                                           bool in_row, int32_t row, int32_t deg, int lane) {
+                                           bool in_row, int lane) {
   const int32_t a = run.x;
   const int32_t len = in_row ? run.y : 0;
   const int32_t incl = wave_incl_scan(len);
@@ -237,15 +281,23 @@ __device__ __forceinline__ void feed_block(WaveSketch<CELLS> &store, RunLookup *
     // Keep the scheduler from hoisting b0's first use above b1's load: the
     // wait for b0 must leave b1 in flight.
     __builtin_amdgcn_sched_barrier(0);
-    feed_batch(store, b0, f0, total, row, deg, lane);
+    st.feed_batch(b0, f0, total, lane);
     b0 = pairs[item_index(lk, len, excl, total, f0 + 2 * kWave, &carry, lane)];
     __builtin_amdgcn_sched_barrier(0);
-    if (f0 + kWave < total) feed_batch(store, b1, f0 + kWave, total, row, deg, lane);
+    if (f0 + kWave < total) st.feed_batch(b1, f0 + kWave, total, lane);
   }
 }
 
-template <int CELLS>
-__global__ void __launch_bounds__(kOvfBlock)
+// Registers: up to capacity 128 at most 64, so that 8 waves share a SIMD, and
+// two fit beside the four of a tier-2 workgroup.
+template <int CELLS> constexpr int ovf_min_waves() {
+  return CELLS <= 4 ? 8 : (CELLS <= 10 ? 5 : 1);
+}
+
+// WIDE: chunks of more than 2^12 rows, whose candidates need a whole word in
+// the counting table.
+template <int CELLS, bool WIDE>
+__global__ void __launch_bounds__(kOvfBlock, (ovf_min_waves<CELLS>()))
     ovf_sketch_kernel(int32_t n, int32_t k, int32_t chunk_size,
                       const int32_t *__restrict__ row_ptr, const int2 *__restrict__ runs,
                       const int2 *__restrict__ pairs, uint64_t *__restrict__ table,
@@ -253,21 +305,34 @@ __global__ void __launch_bounds__(kOvfBlock)
                       const int32_t *__restrict__ list_count, uint32_t *__restrict__ claim,
                       int32_t *__restrict__ row_valid, int64_t l0, int64_t l1) {
   __shared__ RunLookup s_lookup[kOvfWaves];
+  RowStream<CELLS, WIDE> st;
+  __shared__ uint32_t s_count[kOvfWaves][decltype(st.counter)::kWords];
   const int lane = lane_id();
   RunLookup *lk = &s_lookup[threadIdx.x / kWave];
+  st.counter.init(s_count[threadIdx.x / kWave]);
+  st.row_ptr = row_ptr;
   // Rows of list entries [l0, l1); work < 2^32: list_len * chunk_size <=
   // n + chunk_size - 1.
   const int64_t L = range_end(l1, list, list_count, ceil_div64(n, chunk_size));
   const int64_t work = (L > l0 ? L - l0 : 0) * chunk_size;
-  WaveSketch<CELLS> store;
 
-  // Waves claim rows one at a time from a device-wide counter (zeroed by the
-  // host before the launch): a few rows stream millions of items, and a
-  // fixed assignment would give one wave several of them.
-  for (;;) {
-    uint32_t claimed = 0;
-    if (lane == 0) claimed = atomicAdd(claim, 1u);
-    const int64_t w = static_cast<uint32_t>(readlane(static_cast<int32_t>(claimed), 0));
+  // Waves claim rows from a device-wide counter (zeroed by the host before the
+  // launch): a few rows stream millions of items, and a fixed assignment would
+  // give one wave several of them.  A claim takes several rows while many are
+  // left for each wave, at most kClaimRows: one claim after another on the
+  // counter costs about 13 ns, which was all of the time of 262,144 short rows
+  // (3.34 ms with a claim per row).
+  const int64_t waves = static_cast<int64_t>(gridDim.x) * kOvfWaves;
+  int64_t w = 0, w_end = 0; // claimed rows not yet done
+  for (;; ++w) {
+    if (w >= w_end) {
+      int64_t take = (work - w_end) / (2 * waves);
+      take = take < 1 ? 1 : (take > kClaimRows ? kClaimRows : take);
+      uint32_t claimed = 0;
+      if (lane == 0) claimed = atomicAdd(claim, static_cast<uint32_t>(take));
+      w = static_cast<uint32_t>(readlane(static_cast<int32_t>(claimed), 0));
+      w_end = w + take < work ? w + take : work;
+    }
     if (w >= work) break;
     int64_t row64 = l0 * chunk_size + w;
     if (list) {
@@ -283,7 +348,8 @@ __global__ void __launch_bounds__(kOvfBlock)
       if (row_valid != nullptr && lane == 0) row_valid[row] = 0;
       continue;
     }
-    store.clear();
+    st.base = row - row % chunk_size;
+    st.begin(row, deg);
     const int32_t nblk = (deg + kWave - 1) / kWave;
     // Four blocks of runs in flight, each in its own registers (a rotating
     // copy would wait for the loads it copies).
@@ -293,20 +359,20 @@ __global__ void __launch_bounds__(kOvfBlock)
     int2 r3 = load_runs(runs, rs, re, 3, lane);
     for (int32_t blk = 0; blk < nblk; blk += 4) {
       const int64_t p = static_cast<int64_t>(rs) + static_cast<int64_t>(blk) * kWave + lane;
-      feed_block(store, lk, pairs, r0, p < re, row, deg, lane);
+      feed_block(st, lk, pairs, r0, p < re, lane);
       r0 = load_runs(runs, rs, re, blk + 4, lane);
       if (blk + 1 >= nblk) break;
-      feed_block(store, lk, pairs, r1, p + kWave < re, row, deg, lane);
+      feed_block(st, lk, pairs, r1, p + kWave < re, lane);
       r1 = load_runs(runs, rs, re, blk + 5, lane);
       if (blk + 2 >= nblk) break;
-      feed_block(store, lk, pairs, r2, p + 2 * kWave < re, row, deg, lane);
+      feed_block(st, lk, pairs, r2, p + 2 * kWave < re, lane);
       r2 = load_runs(runs, rs, re, blk + 6, lane);
       if (blk + 3 >= nblk) break;
-      feed_block(store, lk, pairs, r3, p + 3 * kWave < re, row, deg, lane);
+      feed_block(st, lk, pairs, r3, p + 3 * kWave < re, lane);
       r3 = load_runs(runs, rs, re, blk + 7, lane);
     }
-    store.select_top_k(k, out);
-    if (row_valid != nullptr && lane == 0) row_valid[row] = min(k, store.filled);
+    st.finish(k, out);
+    if (row_valid != nullptr && lane == 0) row_valid[row] = min(k, st.store.filled);
   }
 }
 
@@ -389,9 +455,10 @@ void launch_ovf_sketch(Context &ctx, int32_t n, int32_t k, int32_t chunk_size,
   // kernels queued beside it).
   const int g = ctx.grid_for(ceil_div64(rows >= 0 ? rows : n, kOvfWaves), kOvfBlock, 4);
   fill_u32(ctx, claim, 1, 0u);
-  ovf_sketch_kernel<CELLS><<<g, kOvfBlock, 0, ctx.stream>>>(n, k, chunk_size, d_ptr, runs,
-                                                            pairs, d_table, list, list_count,
-                                                            claim, d_row_valid, l0, l1);
+  auto *kernel =
+      chunk_size <= 4096 ? ovf_sketch_kernel<CELLS, false> : ovf_sketch_kernel<CELLS, true>;
+  kernel<<<g, kOvfBlock, 0, ctx.stream>>>(n, k, chunk_size, d_ptr, runs, pairs, d_table, list,
+                                          list_count, claim, d_row_valid, l0, l1);
   SP_LAUNCH_CHECK();
 }
 

@@ -525,6 +525,14 @@ template <int CELLS> struct WaveSketch {
         fw[2 * j + 1] = hw;
       }
     }
+    emit_lists(k, out, fk, fw);
+  }
+
+  // select_top_k from the cells of logical lane L in physical lane L (< 32;
+  // the upper half's values are not used).
+  __device__ __forceinline__ void emit_lists(int32_t k, uint64_t *out, int32_t (&fk)[CELLS],
+                                             float (&fw)[CELLS]) {
+    const int lane = lane_id();
     // Selection sort, literally as the reference (not stable).
 #pragma unroll
     for (int i = 0; i < CELLS - 1; ++i) {
@@ -554,9 +562,14 @@ template <int CELLS> struct WaveSketch {
         }
       }
     }
-    if constexpr (CELLS >= 3 && CELLS <= 4) {
-      emit_sorted_lists(k, out, fk, fw);
-      return;
+    // Up to 128 live entries: one sorting network.  The merge below costs
+    // about 45 wave instructions per emitted entry (k = 77 at CELLS = 10: some
+    // 3,500 a row, more than the row's counting; the network about 700).
+    if constexpr (CELLS >= 3) {
+      if (CELLS <= 4 || filled <= 128) {
+        emit_sorted_lists(k, out, fk, fw);
+        return;
+      }
     }
     // k-way merge; lane (i & 63) keeps output entry i in register i >> 6.
     // The row has k <= M = 32 * CELLS <= 64 * LC entries (m = (int)(k * ovs)
@@ -601,8 +614,9 @@ template <int CELLS> struct WaveSketch {
     }
   }
 
-  // The merge of select_top_k for 3 <= CELLS <= 4, from the selection-sorted
-  // lists fk/fw of logical lane L (held by physical lane L < 32).  The merge
+  // The merge of select_top_k for CELLS >= 3 and at most 128 live entries,
+  // from the selection-sorted lists fk/fw of logical lane L (held by physical
+  // lane L < 32).  The merge
   // emits every entry of weight above w before any of weight w (each list
   // descends), and among equal weights drains the smallest logical lane's
   // run first, in list order: output order is (weight descending, L, list
@@ -615,7 +629,7 @@ template <int CELLS> struct WaveSketch {
   __device__ __forceinline__ void emit_sorted_lists(int32_t k, uint64_t *out,
                                                     const int32_t (&fk)[CELLS],
                                                     const float (&fw)[CELLS]) {
-    static_assert(CELLS >= 3 && CELLS <= 4, "two registers of 64 elements");
+    static_assert(CELLS >= 3, "two registers of 64 elements");
     const int lane = lane_id();
     int32_t sk[2];
     uint32_t hi[2], lo[2];
@@ -660,6 +674,7 @@ template <int CELLS> struct WaveSketch {
       const uint64_t v = i < n_live ? pack_wi(idx, __uint_as_float(~hi[q])) : 0ull;
       if (i < k) out[i] = v;
     }
+    for (int32_t i = 2 * kWave + lane; i < k; i += kWave) out[i] = 0;
   }
 
   // select_top_k for CELLS <= 2 (one cell per physical lane).  The merge
@@ -685,6 +700,13 @@ template <int CELLS> struct WaveSketch {
     } else {
       if (lane >= 32) sk = -1;
     }
+    emit_slots(k, out, sk, sw);
+  }
+
+  // The same from slot `lane` in each lane (sk == -1: empty).
+  static __device__ __forceinline__ void emit_slots(int32_t k, uint64_t *out, int32_t sk,
+                                                    float sw) {
+    const int lane = lane_id();
     const bool live = sk != -1;
     const uint64_t lm = ballot(live);
     const int n_live = __popcll(lm);
