@@ -223,7 +223,7 @@ void chunk_sketch_top_k(Context &ctx, int32_t n, int32_t nnz, int32_t k, int32_t
                         const int32_t *d_chunks = nullptr,
                         const int32_t *d_chunk_count = nullptr,
                         hipEvent_t prepared = nullptr, int32_t *d_row_valid = nullptr,
-                        int64_t host_list_len = -1);
+                        int64_t host_list_len = -1, bool count = true);
 // The is_symmetric mirror check of the rows chunk_sketch_top_k computes for
 // the same list: mirror_term (below) of each of their nonzeros, added into
 // *mirror.  Independent of the sketch; the caller runs it where it holds back
@@ -235,14 +235,15 @@ void chunk_mirror_check(Context &ctx, int32_t n, int32_t chunk_size, const int32
 
 // Chunk-local variant: one workgroup per chunk with the chunk's transpose in
 // LDS.  Applicable when chunk_local_supported(n, chunk_size).
-// chunk_local_classify fills d_lists (3*num_chunks int32) and d_counts (4
+// chunk_local_classify fills d_lists (3*num_chunks int32) and d_counts (5
 // int32): the chunks of LDS tier 2 in d_lists[0 .. d_counts[0]), the chunks
 // too large for LDS in d_lists[num_chunks .. num_chunks + d_counts[1]) (for
 // chunk_sketch_top_k over the global CSC; with is_symmetric, the largest
 // chunks that tier 2 could hold go there as well, to run beside it), the
 // tier-1 chunks in d_lists[2 num_chunks .. 2 num_chunks + d_counts[2]), and
 // d_counts[3] = 0, the counter tier 2 claims its chunks from (so each tier-2
-// launch needs a classification before it).  chunk_local_sketch_top_k then
+// launch needs a classification before it), and d_counts[4] = whether rows are
+// to be counted (`count` of the sketch calls).  chunk_local_sketch_top_k then
 // writes the rows of tier-1 chunks (tiers & 1; chunk_size <= 1024) and of the
 // listed tier-2 chunks (tiers & 2); the two launches are independent and may
 // run on different streams.  With t1_list_len >= 0 (d_counts[2], read back)
@@ -251,11 +252,11 @@ void chunk_mirror_check(Context &ctx, int32_t n, int32_t chunk_size, const int32
 constexpr int kLocalRowCap = 4096;
 bool chunk_local_supported(int32_t n, int32_t chunk_size);
 void chunk_local_classify(Context &ctx, int32_t n, int32_t chunk_size, const int32_t *d_ptr,
-                          int32_t *d_lists, int32_t *d_counts, bool is_symmetric);
+                          const int32_t *d_ind, int32_t *d_lists, int32_t *d_counts, bool is_symmetric);
 void chunk_local_sketch_top_k(Context &ctx, int32_t n, int32_t k, int32_t chunk_size,
                               int32_t m_capacity, const int32_t *d_ptr, const int32_t *d_ind,
                               uint64_t *d_table, const int32_t *d_lists,
-                              int32_t *d_counts, int tiers,
+                              int32_t *d_counts, int tiers, bool count,
                               int32_t *d_row_valid = nullptr,
                               unsigned long long *mirror = nullptr,
                               int64_t t1_list_len = -1);

@@ -1215,7 +1215,7 @@ size_t table_ws_bytes(int32_t n, int32_t nnz, int32_t k, int32_t chunk_size,
                       bool is_symmetric) {
   size_t b = ws_bytes<uint64_t>(static_cast<size_t>(n) * k);
   int64_t chunks = ceil_div64(n, chunk_size);
-  b += ws_bytes<int32_t>(3 * static_cast<size_t>(chunks)) + ws_bytes<int32_t>(4);
+  b += ws_bytes<int32_t>(3 * static_cast<size_t>(chunks)) + ws_bytes<int32_t>(5);
   b += chunk_sketch_ws_bytes(n, nnz, chunk_size);
   if (!is_symmetric) {
     b += ws_bytes<int32_t>(static_cast<size_t>(n) + 1) +
@@ -1240,7 +1240,7 @@ void build_table(Context &ctx, int32_t n, int32_t nnz, const int32_t *d_ptr,
                  int32_t *row_valid = nullptr) {
   const int64_t chunks = ceil_div64(n, chunk_size);
   int32_t *lists = ctx.take<int32_t>(3 * static_cast<size_t>(chunks));
-  int32_t *counts = ctx.take<int32_t>(4);
+  int32_t *counts = ctx.take<int32_t>(5);
   const bool local = allow_local && chunk_local_supported(n, chunk_size);
   const bool check_mirror = local && is_symmetric;
   unsigned long long *msum = nullptr;
@@ -1277,7 +1277,8 @@ void build_table(Context &ctx, int32_t n, int32_t nnz, const int32_t *d_ptr,
     return;
   }
 
-  // Chunks are classified and the three list lengths read back; then the
+  // Chunks are classified and the three list lengths (and whether rows are to
+  // be counted) read back; then the
   // sketch paths that have work, which write disjoint table rows, run
   // concurrently: tier 2 (mid-size chunks) on side stream 1, the global-CSC
   // path (large chunks, whose hub rows set the critical path on power-law
@@ -1294,24 +1295,25 @@ void build_table(Context &ctx, int32_t n, int32_t nnz, const int32_t *d_ptr,
   // heaviest chunk's, is queued.  The transpose of a non-symmetric matrix is
   // built only when the global path has chunks.
   t_sim->begin(ctx.stream);
-  chunk_local_classify(ctx, n, chunk_size, d_ptr, lists, counts, is_symmetric);
+  chunk_local_classify(ctx, n, chunk_size, d_ptr, d_ind, lists, counts, is_symmetric);
   int32_t *h_counts = ctx.host_words;
-  SP_HIP(hipMemcpyAsync(h_counts, counts, 3 * sizeof(int32_t), hipMemcpyDeviceToHost,
+  SP_HIP(hipMemcpyAsync(h_counts, counts, 5 * sizeof(int32_t), hipMemcpyDeviceToHost,
                         ctx.stream));
   ctx.sync();
   const bool run_t2 = h_counts[0] > 0, run_global = h_counts[1] > 0;
   const int64_t t1_len = h_counts[2];
+  const bool count = h_counts[4] != 0;
   const bool t1_first = (run_t2 || run_global) && t1_len <= ctx.num_cus;
   if (run_t2) fork_side(ctx, 1);
   if (run_global) fork_side(ctx, 0);
   if (t1_first) {
     chunk_local_sketch_top_k(ctx, n, k, chunk_size, m_cap, d_ptr, d_ind, table, lists, counts,
-                             1, row_valid, msum, t1_len);
+                             1, count, row_valid, msum, t1_len);
   }
   if (run_t2) {
     OnStream on(ctx, ctx.side[1]);
     chunk_local_sketch_top_k(ctx, n, k, chunk_size, m_cap, d_ptr, d_ind, table, lists, counts,
-                             2, row_valid, msum);
+                             2, count, row_valid, msum);
   }
   if (run_global) {
     OnStream on(ctx, ctx.side[0]);
@@ -1321,7 +1323,7 @@ void build_table(Context &ctx, int32_t n, int32_t nnz, const int32_t *d_ptr,
     t_csc->end(ctx.stream);
     chunk_sketch_top_k(ctx, n, nnz, k, chunk_size, m_cap, d_ptr, d_ind, cp, ri, table,
                        lists + chunks, counts + 1, t1_first ? nullptr : ctx.prep_ev, row_valid,
-                       h_counts[1]);
+                       h_counts[1], count);
   } else {
     t_csc->begin(ctx.stream);
     t_csc->end(ctx.stream);
@@ -1329,7 +1331,7 @@ void build_table(Context &ctx, int32_t n, int32_t nnz, const int32_t *d_ptr,
   if (!t1_first) {
     if (run_global) SP_HIP(hipStreamWaitEvent(ctx.stream, ctx.prep_ev, 0));
     chunk_local_sketch_top_k(ctx, n, k, chunk_size, m_cap, d_ptr, d_ind, table, lists, counts,
-                             1, row_valid, msum);
+                             1, count, row_valid, msum);
   }
   // The global path's rows' mirror check, behind tier 1 on the library
   // stream: ahead of the global path's other chunks (on side stream 2) it held

@@ -37,7 +37,7 @@
 // sketch before): random geometric graph of 2^20 points, mean degree 13, 79
 // items a row: 2.23 -> 1.34 ms; planted blocks of 600,000 rows of 22 in block
 // order, 400 items a row: 7.92 -> 3.06 ms; a scrambled matrix whose rows have
-// hardly an item: 0.267 -> 0.274 ms (16-bit bucket ends, a larger kernel).
+// hardly an item: 0.263 -> 0.265 ms (not counted: sample_shared).
 // Larger chunks go to an overflow list for the global-CSC kernel.  Requires
 // ceil(log2 n) + ceil(log2 C) <= 32 (checked by the host).
 #include "common.hpp"
@@ -177,7 +177,9 @@ template <int CELLS, int KEYCAP, int ROWCAP, int NB> struct LocalLds {
   uint16_t order[ROWCAP];
 };
 
-template <int CELLS, int KEYCAP, int ROWCAP, int NB_LOG2, bool CLAIM>
+// COUNT: rows are counted while they need no eviction (sample_shared below
+// says when); false feeds every item to the sketch.
+template <int CELLS, int KEYCAP, int ROWCAP, int NB_LOG2, bool CLAIM, bool COUNT>
 __global__ void __launch_bounds__(kLocalThreads)
     __attribute__((amdgpu_waves_per_eu(local_eu_waves<CELLS, KEYCAP>())))
     chunk_local_sketch_kernel(int32_t n, int32_t k, int32_t chunk_size, int32_t lb,
@@ -226,7 +228,7 @@ __global__ void __launch_bounds__(kLocalThreads)
   const int64_t work = chunk_list ? *chunk_list_count : num_chunks;
 
   typename Lds::Counter counter;
-  counter.init(lds.count[wave]);
+  if constexpr (COUNT) counter.init(lds.count[wave]);
   if (lane == 0) lds.starts[wave] = 0;
   for (int32_t r = threadIdx.x; r < ROWCAP; r += kLocalThreads) s_order[r] = 0;
   if (threadIdx.x == 0) s_mirror = 0;
@@ -558,10 +560,10 @@ __global__ void __launch_bounds__(kLocalThreads)
       // made the first slower (csg of 20,000 rows of 10: 0.52 -> 0.54 ms).
       int32_t pb = rb, f0 = 0; // where the item-by-item form begins
       // Each of the row's own columns holds the row itself, which is no item.
-      bool serial = row_size <= kWave && total - row_size <= kSerialItems;
+      bool serial = !COUNT || (row_size <= kWave && total - row_size <= kSerialItems);
       if (serial) {
         store.clear();
-      } else {
+      } else if constexpr (COUNT) {
         // Counted 64 items at a time while the row needs no eviction; after
         // that it goes on item by item from its counts, or starts again.
         bool go_on = false, again = false;
@@ -664,6 +666,40 @@ __device__ __forceinline__ int tier_list(int tier) {
   return tier == 1 ? 2 : (tier >= 2 ? tier - 2 : -1);
 }
 
+// Whether the sketch kernels count rows (row_count.hpp), which only pays where
+// rows meet few others often: what tells is whether neighbouring rows share
+// columns.  Samples kClassifyThreads / 16 places of a row and the one after it,
+// 16 lanes each: of the first 16 nonzeros of the row, how many are among the
+// first 16 of the next.  At least an eighth (7-point stencil 0.29, blocks of 64
+// rows 0.2, geometric graphs and finite elements about a half): the counting
+// kernels.  Fewer (power-law graphs 0.02-0.06, scrambled matrices 0): rows have
+// hardly an item or evict all along, and kernels without the counting form,
+// which spill less, are faster there (reorder, apply and SpMM of a power-law
+// graph, 153,000 rows of 22: 7.49 ms counted, 6.69 not; csg of one of 2.4 M
+// rows of 25: 19.2 and 18.3 ms).  The table is the same either way.
+__device__ __forceinline__ void sample_shared(int32_t n, const int32_t *__restrict__ row_ptr,
+                                              const int32_t *__restrict__ col_ind,
+                                              int32_t *shared, int32_t *seen) {
+  constexpr int kGroup = 16, kPlaces = kClassifyThreads / kGroup;
+  if (n < 2) return;
+  const int lane = lane_id(), gl = lane & (kGroup - 1);
+  const int64_t place = threadIdx.x / kGroup;
+  const int64_t r = (2 * place + 1) * (n - 1) / (2 * kPlaces); // at most n - 2
+  const int32_t a = row_ptr[r], b = row_ptr[r + 1], c = row_ptr[r + 2];
+  const int32_t mine = gl < b - a ? col_ind[a + gl] : -1;
+  const int32_t next = gl < c - b ? col_ind[b + gl] : -2;
+  bool found = false;
+#pragma unroll
+  for (int i = 0; i < kGroup; ++i) {
+    found |= mine == __shfl(next, (lane & ~(kGroup - 1)) + i, kWave);
+  }
+  const int32_t nf = __popcll(ballot(found)), ns = __popcll(ballot(mine >= 0));
+  if (lane == 0) {
+    atomicAdd(shared, nf);
+    atomicAdd(seen, ns);
+  }
+}
+
 // Lists the chunks by tier: tier-2 chunks in lists[0 .. counts[0]),
 // global-path chunks in lists[chunks .. chunks + counts[1]), tier-1 chunks in
 // lists[2 chunks .. 2 chunks + counts[2]); counts[3] = 0 (the counter tier 2
@@ -677,12 +713,21 @@ __device__ __forceinline__ int tier_list(int tier) {
 // table does not depend on list order.
 __global__ void __launch_bounds__(kClassifyThreads)
     classify_chunks_kernel(int32_t n, int32_t chunk_size, int t1, int32_t t2_keys,
-                           const int32_t *__restrict__ row_ptr, int32_t *__restrict__ lists,
+                           const int32_t *__restrict__ row_ptr,
+                           const int32_t *__restrict__ col_ind, int32_t *__restrict__ lists,
                            int32_t *__restrict__ counts) {
   __shared__ int32_t s_cls[2][kClasses + 1];
   __shared__ int32_t s_t1;
+  __shared__ int32_t s_shared, s_seen;
   const int64_t chunks = ceil_div64(n, chunk_size);
   const int tid = threadIdx.x, lane = lane_id();
+  if (blockIdx.x == 0) {
+    if (tid == 0) s_shared = s_seen = 0;
+    __syncthreads();
+    sample_shared(n, row_ptr, col_ind, &s_shared, &s_seen);
+    __syncthreads();
+    if (tid == 0) counts[4] = 8 * s_shared >= s_seen ? 1 : 0;
+  }
   auto chunk_of = [&](int64_t q, int32_t *E) {
     const int64_t cs = q * chunk_size;
     const int64_t ce = cs + chunk_size < n ? cs + chunk_size : n;
@@ -759,7 +804,7 @@ __global__ void __launch_bounds__(kClassifyThreads)
   }
 }
 
-template <int CELLS, int KEYCAP, int ROWCAP, int NB_LOG2, bool CLAIM>
+template <int CELLS, int KEYCAP, int ROWCAP, int NB_LOG2, bool CLAIM, bool COUNT>
 void launch_tier(Context &ctx, int32_t n, int32_t k, int32_t chunk_size, int32_t lb,
                  const int32_t *d_ptr, const int32_t *d_ind, uint64_t *d_table,
                  const int32_t *list, const int32_t *list_count, int64_t host_len,
@@ -775,7 +820,7 @@ void launch_tier(Context &ctx, int32_t n, int32_t k, int32_t chunk_size, int32_t
   if (grid <= 0) return;
   using Lds = LocalLds<CELLS, KEYCAP, ROWCAP, 1 << NB_LOG2>;
   static_assert(sizeof(Lds) <= (KEYCAP <= 16384 ? 80 : 160) * 1024, "workgroups per CU");
-  chunk_local_sketch_kernel<CELLS, KEYCAP, ROWCAP, NB_LOG2, CLAIM>
+  chunk_local_sketch_kernel<CELLS, KEYCAP, ROWCAP, NB_LOG2, CLAIM, COUNT>
       <<<dim3(static_cast<unsigned>(grid)), kLocalThreads, sizeof(Lds), ctx.stream>>>(
           n, k, chunk_size, lb, d_ptr, d_ind, d_table, list, list_count, ovf, ovf_count,
           d_row_valid, mirror, claim);
@@ -785,18 +830,21 @@ void launch_tier(Context &ctx, int32_t n, int32_t k, int32_t chunk_size, int32_t
 template <int CELLS>
 void launch_local(Context &ctx, int32_t n, int32_t k, int32_t chunk_size, int32_t lb,
                   const int32_t *d_ptr, const int32_t *d_ind, uint64_t *d_table,
-                  const int32_t *lists, int32_t *counts, int tiers, int64_t t1_list_len,
+                  const int32_t *lists, int32_t *counts, int tiers, bool count, int64_t t1_list_len,
                   int32_t *d_row_valid, unsigned long long *mirror) {
   const int64_t chunks = ceil_div64(n, chunk_size);
   if (tiers & 2) {
-    auto *tier2 = chunk_size <= kT1Rows ? launch_tier<CELLS, kT2Keys, kT1Rows, kT2Nb, true>
-                                        : launch_tier<CELLS, kT2Keys, kT2Rows, kT2Nb, true>;
+    auto *tier2 = !count ? launch_tier<CELLS, kT2Keys, kT2Rows, kT2Nb, true, false>
+                  : chunk_size <= kT1Rows ? launch_tier<CELLS, kT2Keys, kT1Rows, kT2Nb, true, true>
+                                          : launch_tier<CELLS, kT2Keys, kT2Rows, kT2Nb, true, true>;
     tier2(ctx, n, k, chunk_size, lb, d_ptr, d_ind, d_table, lists, counts, -1, nullptr, nullptr,
           1, d_row_valid, mirror, reinterpret_cast<uint32_t *>(counts + 3));
   }
   if ((tiers & 1) && chunk_size <= kT1Rows) {
     const bool listed = t1_list_len >= 0;
-    launch_tier<CELLS, kT1Keys, kT1Rows, kT1Nb, false>(
+    auto *tier1 = count ? launch_tier<CELLS, kT1Keys, kT1Rows, kT1Nb, false, true>
+                        : launch_tier<CELLS, kT1Keys, kT1Rows, kT1Nb, false, false>;
+    tier1(
         ctx, n, k, chunk_size, lb, d_ptr, d_ind, d_table, listed ? lists + 2 * chunks : nullptr,
         listed ? counts + 2 : nullptr, t1_list_len, nullptr, nullptr, 2, d_row_valid, mirror,
         nullptr);
@@ -810,25 +858,26 @@ bool chunk_local_supported(int32_t n, int32_t chunk_size) {
 }
 
 void chunk_local_classify(Context &ctx, int32_t n, int32_t chunk_size, const int32_t *d_ptr,
-                          int32_t *d_lists, int32_t *d_counts, bool is_symmetric) {
+                          const int32_t *d_ind, int32_t *d_lists, int32_t *d_counts,
+                          bool is_symmetric) {
   SP_EXPECT(chunk_local_supported(n, chunk_size), "chunk-local sketch not applicable");
   const int64_t chunks = ceil_div64(n, chunk_size);
   const int t1 = chunk_size <= kT1Rows ? 1 : 0;
   int grid = 1;
   if (chunks > kClassifyOrderCap) {
     grid = ctx.grid_for(ceil_div64(chunks, kClassifyThreads), kClassifyThreads, 1);
-    fill_u32(ctx, d_counts, 4, 0u);
+    fill_u32(ctx, d_counts, 5, 0u);
   }
   const int32_t t2_keys = is_symmetric ? kT2SharedKeys : kT2Keys;
   classify_chunks_kernel<<<grid, kClassifyThreads, 0, ctx.stream>>>(n, chunk_size, t1, t2_keys,
-                                                                    d_ptr, d_lists, d_counts);
+                                                                    d_ptr, d_ind, d_lists, d_counts);
   SP_LAUNCH_CHECK();
 }
 
 void chunk_local_sketch_top_k(Context &ctx, int32_t n, int32_t k, int32_t chunk_size,
                               int32_t m_capacity, const int32_t *d_ptr, const int32_t *d_ind,
                               uint64_t *d_table, const int32_t *d_lists,
-                              int32_t *d_counts, int tiers, int32_t *d_row_valid,
+                              int32_t *d_counts, int tiers, bool count, int32_t *d_row_valid,
                               unsigned long long *mirror, int64_t t1_list_len) {
   SP_EXPECT(k <= 512, "k must be <= 512");
   SP_EXPECT(chunk_local_supported(n, chunk_size), "chunk-local sketch not applicable");
@@ -837,7 +886,7 @@ void chunk_local_sketch_top_k(Context &ctx, int32_t n, int32_t k, int32_t chunk_
 #define SP_CASE(C)                                                                       \
   case C:                                                                                \
     launch_local<C>(ctx, n, k, chunk_size, lb, d_ptr, d_ind, d_table, d_lists, d_counts, \
-                    tiers, t1_list_len, d_row_valid, mirror);                            \
+                    tiers, count, t1_list_len, d_row_valid, mirror);                     \
     break;
     SP_CASE(1) SP_CASE(2) SP_CASE(3) SP_CASE(4) SP_CASE(5) SP_CASE(6)
     SP_CASE(7) SP_CASE(8) SP_CASE(9) SP_CASE(10) SP_CASE(11) SP_CASE(12)

@@ -216,7 +216,7 @@ __device__ __forceinline__ int32_t item_index(RunLookup *lk, int32_t len, int32_
 
 // One row's stream: counted 64 items at a time (row_count.hpp) while it needs
 // no eviction, item by item in the sketch afterwards.
-template <int CELLS, bool WIDE> struct RowStream {
+template <int CELLS, bool WIDE, bool COUNT> struct RowStream {
   RowCounter<CELLS, row_table_entries(32 * CELLS), WIDE> counter;
   WaveSketch<CELLS> store;
   bool counting, opening; // wave-uniform; opening: no batch taken yet
@@ -227,37 +227,42 @@ template <int CELLS, bool WIDE> struct RowStream {
   __device__ __forceinline__ void begin(int32_t r, int32_t d) {
     row = r;
     deg = d;
-    counting = true;
+    counting = COUNT;
     opening = true;
+    if constexpr (!COUNT) store.clear();
   }
   __device__ __forceinline__ int32_t size_of(int32_t s) const {
     return row_ptr[s + 1] - row_ptr[s];
   }
   __device__ __forceinline__ void feed_batch(int2 pr, int32_t f0, int32_t total, int lane) {
     const uint64_t items = ballot(f0 + lane < total && pr.x != row);
-    if (counting && opening) {
-      opening = false;
-      if (counter.add(items, static_cast<uint32_t>(pr.x - base)) &&
-          !counter.will_evict(total)) {
-        return;
+    if constexpr (COUNT) {
+      if (counting && opening) {
+        opening = false;
+        if (counter.add(items, static_cast<uint32_t>(pr.x - base)) &&
+            !counter.will_evict(total)) {
+          return;
+        }
+        // Evictions at once or ahead: this batch again, item by item.
+        counter.empty();
+        store.clear();
+        counting = false;
+      } else if (counting) {
+        if (counter.add(items, static_cast<uint32_t>(pr.x - base))) return;
+        counter.to_sketch(store, base, deg, [this](int32_t s) { return size_of(s); });
+        counting = false;
       }
-      // Evictions at once or ahead: this batch again, item by item.
-      counter.empty();
-      store.clear();
-      counting = false;
-    } else if (counting) {
-      if (counter.add(items, static_cast<uint32_t>(pr.x - base))) return;
-      counter.to_sketch(store, base, deg, [this](int32_t s) { return size_of(s); });
-      counting = false;
     }
     store.feed(items, pr.x, 2.0f / static_cast<float>(deg + pr.y));
   }
   __device__ __forceinline__ void finish(int32_t k, uint64_t *out) {
-    if (counting) {
-      counter.emit(store, k, out, base, deg, [this](int32_t s) { return size_of(s); });
-    } else {
-      store.select_top_k(k, out);
+    if constexpr (COUNT) {
+      if (counting) {
+        counter.emit(store, k, out, base, deg, [this](int32_t s) { return size_of(s); });
+        return;
+      }
     }
+    store.select_top_k(k, out);
   }
 };
 
@@ -288,16 +293,18 @@ __device__ __forceinline__ void feed_block(Stream &st, RunLookup *lk,
   }
 }
 
-// Registers: up to capacity 128 at most 64, so that 8 waves share a SIMD, and
-// two fit beside the four of a tier-2 workgroup.
-template <int CELLS> constexpr int ovf_min_waves() {
-  return CELLS <= 4 ? 8 : (CELLS <= 10 ? 5 : 1);
+// Registers: with counting, up to capacity 128 at most 64, so that 8 waves
+// share a SIMD, and two fit beside the four of a tier-2 workgroup; without it
+// the kernel needs 33 to 62 by itself.
+template <int CELLS, bool COUNT> constexpr int ovf_min_waves() {
+  return !COUNT ? 1 : (CELLS <= 4 ? 8 : (CELLS <= 10 ? 5 : 1));
 }
 
 // WIDE: chunks of more than 2^12 rows, whose candidates need a whole word in
-// the counting table.
-template <int CELLS, bool WIDE>
-__global__ void __launch_bounds__(kOvfBlock, (ovf_min_waves<CELLS>()))
+// the counting table.  COUNT: rows are counted (sample_shared in csg_local.hip);
+// false feeds every item to the sketch.
+template <int CELLS, bool WIDE, bool COUNT>
+__global__ void __launch_bounds__(kOvfBlock, (ovf_min_waves<CELLS, COUNT>()))
     ovf_sketch_kernel(int32_t n, int32_t k, int32_t chunk_size,
                       const int32_t *__restrict__ row_ptr, const int2 *__restrict__ runs,
                       const int2 *__restrict__ pairs, uint64_t *__restrict__ table,
@@ -305,11 +312,11 @@ __global__ void __launch_bounds__(kOvfBlock, (ovf_min_waves<CELLS>()))
                       const int32_t *__restrict__ list_count, uint32_t *__restrict__ claim,
                       int32_t *__restrict__ row_valid, int64_t l0, int64_t l1) {
   __shared__ RunLookup s_lookup[kOvfWaves];
-  RowStream<CELLS, WIDE> st;
-  __shared__ uint32_t s_count[kOvfWaves][decltype(st.counter)::kWords];
+  RowStream<CELLS, WIDE, COUNT> st;
+  __shared__ uint32_t s_count[kOvfWaves][COUNT ? decltype(st.counter)::kWords : 1];
   const int lane = lane_id();
   RunLookup *lk = &s_lookup[threadIdx.x / kWave];
-  st.counter.init(s_count[threadIdx.x / kWave]);
+  if constexpr (COUNT) st.counter.init(s_count[threadIdx.x / kWave]);
   st.row_ptr = row_ptr;
   // Rows of list entries [l0, l1); work < 2^32: list_len * chunk_size <=
   // n + chunk_size - 1.
@@ -448,15 +455,16 @@ void launch_ovf_sketch(Context &ctx, int32_t n, int32_t k, int32_t chunk_size,
                        const int32_t *d_ptr, const int2 *runs, const int2 *pairs,
                        uint64_t *d_table, const int32_t *list, const int32_t *list_count,
                        uint32_t *claim, int32_t *d_row_valid, int64_t l0, int64_t l1,
-                       int64_t rows) {
+                       int64_t rows, bool count) {
   // A wave per row at most: rows = the launch's row slots when the host knows
   // them (a grid sized for every row of the matrix made a one-chunk launch
   // dispatch thousands of workgroups that found no row, holding back the
   // kernels queued beside it).
   const int g = ctx.grid_for(ceil_div64(rows >= 0 ? rows : n, kOvfWaves), kOvfBlock, 4);
   fill_u32(ctx, claim, 1, 0u);
-  auto *kernel =
-      chunk_size <= 4096 ? ovf_sketch_kernel<CELLS, false> : ovf_sketch_kernel<CELLS, true>;
+  auto *kernel = !count ? ovf_sketch_kernel<CELLS, false, false>
+                 : chunk_size <= 4096 ? ovf_sketch_kernel<CELLS, false, true>
+                                      : ovf_sketch_kernel<CELLS, true, true>;
   kernel<<<g, kOvfBlock, 0, ctx.stream>>>(n, k, chunk_size, d_ptr, runs, pairs, d_table, list,
                                           list_count, claim, d_row_valid, l0, l1);
   SP_LAUNCH_CHECK();
@@ -488,7 +496,7 @@ void chunk_sketch_top_k(Context &ctx, int32_t n, int32_t nnz, int32_t k, int32_t
                         const int32_t *d_col_ptr, const int32_t *d_row_ind,
                         uint64_t *d_table, const int32_t *d_chunks,
                         const int32_t *d_chunk_count, hipEvent_t prepared,
-                        int32_t *d_row_valid, int64_t host_list_len) {
+                        int32_t *d_row_valid, int64_t host_list_len, bool count) {
   SP_EXPECT(k <= 512, "k must be <= 512");
   SP_EXPECT(m_capacity % 32 == 0 && m_capacity >= 32 && m_capacity <= 512,
             "sketch capacity must be a multiple of 32 in [32, 512]");
@@ -527,7 +535,7 @@ void chunk_sketch_top_k(Context &ctx, int32_t n, int32_t nnz, int32_t k, int32_t
 #define SP_CASE(C)                                                                         \
   case C:                                                                                  \
     launch_ovf_sketch<C>(ctx, n, k, chunk_size, d_ptr, runs, pairs, d_table, d_chunks,     \
-                         d_chunk_count, cl, d_row_valid, l0, l1, rows);                    \
+                         d_chunk_count, cl, d_row_valid, l0, l1, rows, count);             \
     break;
       SP_CASE(1) SP_CASE(2) SP_CASE(3) SP_CASE(4) SP_CASE(5) SP_CASE(6)
       SP_CASE(7) SP_CASE(8) SP_CASE(9) SP_CASE(10) SP_CASE(11) SP_CASE(12)
