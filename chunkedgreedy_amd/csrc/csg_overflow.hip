@@ -27,9 +27,10 @@
 //      ahead, counting them in LDS while the row needs no eviction
 //      (row_count.hpp) and feeding the wave64 space-saving sketch (sketch.hpp)
 //      otherwise.  Finite-element matrix of 192,000 rows of 77 nonzeros (2,200
-//      items a row, capacity 320): the sketch 13.0 -> 2.6 ms; global sketch of
-//      a 2^18-point geometric graph: 3.34 -> 2.33 ms.  An item's
-//      run is found by marking run starts in LDS and a DPP running maximum.
+//      items a row, capacity 320): the sketch 13.0 -> 2.1 ms; global sketch of
+//      a 2^18-point geometric graph: 3.34 -> 0.57 ms (both with the counters
+//      that rows are claimed from).  An item's run is found by marking run
+//      starts in LDS and a DPP running maximum.
 // The stream, and therefore the table, is the reference's.
 #include "common.hpp"
 #include "row_count.hpp"
@@ -48,7 +49,11 @@ constexpr int kOvfBlock = 256;
 constexpr int kOvfWaves = kOvfBlock / kWave;
 constexpr int kMirrorBlock = 256;
 constexpr int kMirrorRowCap = 64; // longer rows: the whole wave (ovf_mirror_kernel)
-constexpr int kClaimRows = 16;   // most rows of one claim (ovf_sketch_kernel)
+// Row claims (ovf_sketch_kernel): a counter per XCD, 256 bytes apart, each for
+// every kXcds-th run of kClaimRun rows.
+constexpr int kClaimRun = 16;
+constexpr int kClaimStride = 64;
+constexpr int kClaimWords = kXcds * kClaimStride;
 constexpr int kSample = 16;      // run-search sample stride (one 64-byte line)
 
 __device__ __forceinline__ int64_t list_len(const int32_t *list, const int32_t *list_count,
@@ -323,24 +328,26 @@ __global__ void __launch_bounds__(kOvfBlock, (ovf_min_waves<CELLS, COUNT>()))
   const int64_t L = range_end(l1, list, list_count, ceil_div64(n, chunk_size));
   const int64_t work = (L > l0 ? L - l0 : 0) * chunk_size;
 
-  // Waves claim rows from a device-wide counter (zeroed by the host before the
-  // launch): a few rows stream millions of items, and a fixed assignment would
-  // give one wave several of them.  A claim takes several rows while many are
-  // left for each wave, at most kClaimRows: one claim after another on the
-  // counter costs about 13 ns, which was all of the time of 262,144 short rows
-  // (3.34 ms with a claim per row).
-  const int64_t waves = static_cast<int64_t>(gridDim.x) * kOvfWaves;
-  int64_t w = 0, w_end = 0; // claimed rows not yet done
-  for (;; ++w) {
-    if (w >= w_end) {
-      int64_t take = (work - w_end) / (2 * waves);
-      take = take < 1 ? 1 : (take > kClaimRows ? kClaimRows : take);
-      uint32_t claimed = 0;
-      if (lane == 0) claimed = atomicAdd(claim, static_cast<uint32_t>(take));
-      w = static_cast<uint32_t>(readlane(static_cast<int32_t>(claimed), 0));
-      w_end = w + take < work ? w + take : work;
+  // Waves claim rows one at a time (counters zeroed by the host before the
+  // launch): a few rows stream millions of items, and a fixed assignment, or a
+  // claim of several neighbouring rows, would give one wave several of them
+  // (16 rows of 20,000 nonzeros ahead of 1.2 M short ones: 165 ms when a claim
+  // took up to 16 rows).  Claims on one counter follow each other 13 ns apart,
+  // which was all of the time of 262,144 short rows (3.34 ms; 0.57 ms now), so
+  // there is a counter per XCD, and a wave whose own has no row left goes on to
+  // the next one's.  A counter hands out runs of kClaimRun rows, so that neighbouring
+  // rows, which share columns, stay on one XCD's L2.
+  int s = blockIdx.x % kXcds;
+  for (int done = 0;;) {
+    uint32_t claimed = 0;
+    if (lane == 0) claimed = atomicAdd(&claim[s * kClaimStride], 1u);
+    const int64_t c = static_cast<uint32_t>(readlane(static_cast<int32_t>(claimed), 0));
+    const int64_t w = (c / kClaimRun * kXcds + s) * kClaimRun + c % kClaimRun;
+    if (w >= work) {
+      if (++done == kXcds) break;
+      s = (s + 1) % kXcds;
+      continue;
     }
-    if (w >= work) break;
     int64_t row64 = l0 * chunk_size + w;
     if (list) {
       row64 = static_cast<int64_t>(list[l0 + w / chunk_size]) * chunk_size + (w % chunk_size);
@@ -459,9 +466,12 @@ void launch_ovf_sketch(Context &ctx, int32_t n, int32_t k, int32_t chunk_size,
   // A wave per row at most: rows = the launch's row slots when the host knows
   // them (a grid sized for every row of the matrix made a one-chunk launch
   // dispatch thousands of workgroups that found no row, holding back the
-  // kernels queued beside it).
-  const int g = ctx.grid_for(ceil_div64(rows >= 0 ? rows : n, kOvfWaves), kOvfBlock, 4);
-  fill_u32(ctx, claim, 1, 0u);
+  // kernels queued beside it).  No more workgroups than the device holds: a
+  // later one would only ask every counter in vain (four times as many: csg of
+  // the finite-element matrix 4.0 -> 4.3 ms, cg of the geometric graph 1.3 ->
+  // 1.6).
+  const int g = ctx.grid_for(ceil_div64(rows >= 0 ? rows : n, kOvfWaves), kOvfBlock, 1);
+  fill_u32(ctx, claim, kClaimWords, 0u);
   auto *kernel = !count ? ovf_sketch_kernel<CELLS, false, false>
                  : chunk_size <= 4096 ? ovf_sketch_kernel<CELLS, false, true>
                                       : ovf_sketch_kernel<CELLS, true, true>;
@@ -488,7 +498,7 @@ void chunk_mirror_check(Context &ctx, int32_t n, int32_t chunk_size, const int32
 size_t chunk_sketch_ws_bytes(int32_t n, int32_t nnz, int32_t chunk_size) {
   return 2 * ws_bytes<int2>(static_cast<size_t>(nnz)) +
          ws_bytes<int32_t>(static_cast<size_t>(ceil_div64(n, chunk_size)) + 1) +
-         ws_bytes<uint32_t>(2) + ws_bytes<int32_t>(static_cast<size_t>(nnz) / kSample + 1);
+         ws_bytes<uint32_t>(2 * kClaimWords) + ws_bytes<int32_t>(static_cast<size_t>(nnz) / kSample + 1);
 }
 
 void chunk_sketch_top_k(Context &ctx, int32_t n, int32_t nnz, int32_t k, int32_t chunk_size,
@@ -504,7 +514,7 @@ void chunk_sketch_top_k(Context &ctx, int32_t n, int32_t nnz, int32_t k, int32_t
   int2 *runs = ctx.take<int2>(static_cast<size_t>(nnz));
   int2 *pairs = ctx.take<int2>(static_cast<size_t>(nnz));
   int32_t *task_off = ctx.take<int32_t>(static_cast<size_t>(chunks) + 1);
-  uint32_t *claim = ctx.take<uint32_t>(2);
+  uint32_t *claim = ctx.take<uint32_t>(2 * kClaimWords);
   int32_t *sample = ctx.take<int32_t>(static_cast<size_t>(nnz) / kSample + 1);
 
   ovf_plan_kernel<<<1, kPlanBlock, 0, ctx.stream>>>(n, chunk_size, d_ptr, d_chunks,
@@ -565,7 +575,7 @@ void chunk_sketch_top_k(Context &ctx, int32_t n, int32_t nnz, int32_t k, int32_t
     OnStream on(ctx, ctx.side[2]);
     runs_launch(1, -1);
     if (prepared != nullptr) SP_HIP(hipEventRecord(prepared, ctx.stream));
-    sketch_launch(claim + 1, 1, -1);
+    sketch_launch(claim + kClaimWords, 1, -1);
   }
   join_side(ctx, 2);
 }
