@@ -204,6 +204,11 @@ size_t csr2csc_ws_bytes(int32_t n, int32_t nnz);
 void csr2csc(Context &ctx, int32_t n, int32_t nnz, const int32_t *d_ptr,
              const int32_t *d_ind, int32_t *d_col_ptr, int32_t *d_row_ind);
 
+// Whether the sketch counts rows (row_count.hpp): as the classification found
+// (chunk_local_classify), or, where no chunks were classified, as a sample of
+// the rows tells on the device.
+enum class CountRows { kNo, kYes, kSampled };
+
 // Chunk-restricted sketch + top-k table (u64 weighted_index, n*k) from the
 // global CSC.  With d_chunks non-null only the rows of the chunks listed in
 // d_chunks[0 .. *d_chunk_count) are computed.  `prepared`, when given, is
@@ -215,15 +220,15 @@ void csr2csc(Context &ctx, int32_t n, int32_t nnz, const int32_t *d_ptr,
 // size class) have its run search and sketch first while the other chunks'
 // run search runs beside it on side stream 2 (joined back before return).
 // Must be called with ctx.stream = side[0] or the library stream, not side[2].
+// `count` is kSampled if and only if d_chunks is null.
 size_t chunk_sketch_ws_bytes(int32_t n, int32_t nnz, int32_t chunk_size);
 void chunk_sketch_top_k(Context &ctx, int32_t n, int32_t nnz, int32_t k, int32_t chunk_size,
                         int32_t m_capacity, const int32_t *d_ptr,
                         const int32_t *d_ind, const int32_t *d_col_ptr,
                         const int32_t *d_row_ind, uint64_t *d_table,
-                        const int32_t *d_chunks = nullptr,
-                        const int32_t *d_chunk_count = nullptr,
-                        hipEvent_t prepared = nullptr, int32_t *d_row_valid = nullptr,
-                        int64_t host_list_len = -1, bool count = true);
+                        const int32_t *d_chunks, const int32_t *d_chunk_count,
+                        hipEvent_t prepared, int32_t *d_row_valid, int64_t host_list_len,
+                        CountRows count);
 // The is_symmetric mirror check of the rows chunk_sketch_top_k computes for
 // the same list: mirror_term (below) of each of their nonzeros, added into
 // *mirror.  Independent of the sketch; the caller runs it where it holds back

@@ -1272,7 +1272,7 @@ void build_table(Context &ctx, int32_t n, int32_t nnz, const int32_t *d_ptr,
     t_csc->end(ctx.stream);
     t_sim->begin(ctx.stream);
     chunk_sketch_top_k(ctx, n, nnz, k, chunk_size, m_cap, d_ptr, d_ind, cp, ri, table,
-                       nullptr, nullptr, nullptr, row_valid);
+                       nullptr, nullptr, nullptr, row_valid, -1, CountRows::kSampled);
     t_sim->end(ctx.stream);
     return;
   }
@@ -1323,7 +1323,7 @@ void build_table(Context &ctx, int32_t n, int32_t nnz, const int32_t *d_ptr,
     t_csc->end(ctx.stream);
     chunk_sketch_top_k(ctx, n, nnz, k, chunk_size, m_cap, d_ptr, d_ind, cp, ri, table,
                        lists + chunks, counts + 1, t1_first ? nullptr : ctx.prep_ev, row_valid,
-                       h_counts[1], count);
+                       h_counts[1], count ? CountRows::kYes : CountRows::kNo);
   } else {
     t_csc->begin(ctx.stream);
     t_csc->end(ctx.stream);

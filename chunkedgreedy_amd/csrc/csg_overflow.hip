@@ -55,6 +55,7 @@ constexpr int kClaimRun = 16;
 constexpr int kClaimStride = 64;
 constexpr int kClaimWords = kXcds * kClaimStride;
 constexpr int kSample = 16;      // run-search sample stride (one 64-byte line)
+constexpr int kSampleRows = 256; // rows that ovf_sample_kernel looks at
 
 __device__ __forceinline__ int64_t list_len(const int32_t *list, const int32_t *list_count,
                                             int64_t num_chunks) {
@@ -298,6 +299,58 @@ __device__ __forceinline__ void feed_block(Stream &st, RunLookup *lk,
   }
 }
 
+// Whether rows are to be counted where the chunks were not classified: the
+// first block of 64 runs of kSampleRows rows, evenly spaced, a wave each.
+// weight[0] is the sum of their items, weight[1] of those in rows that will
+// likely evict (evicts_soon).  Rows that evict all along gain nothing from
+// counting and pay for its table and registers: cg of a power-law graph of
+// 150,000 rows, capacity 512: 264 ms counted, 217 not; chunks of 20,000 rows of
+// one of 600,000: 152 and 124.  That neighbouring rows share no columns
+// (sample_shared) does not tell here, where a row meets the whole matrix:
+// scrambled blocks of 64 rows, 600,000 rows of 14, capacity 256: 5.5 ms
+// counted, 8.9 not.
+__global__ void __launch_bounds__(kOvfBlock)
+    ovf_sample_kernel(int32_t n, int32_t capacity, const int32_t *__restrict__ row_ptr,
+                      const int2 *__restrict__ runs, const int2 *__restrict__ pairs,
+                      uint32_t *__restrict__ weight) {
+  __shared__ RunLookup s_lookup[kOvfWaves];
+  const int lane = lane_id();
+  RunLookup *lk = &s_lookup[threadIdx.x / kWave];
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kOvfWaves + threadIdx.x / kWave;
+  const int32_t row = static_cast<int32_t>((2 * i + 1) * n / (2 * kSampleRows)); // below n
+  const int32_t rs = row_ptr[row], re = row_ptr[row + 1];
+  if (rs == re) return;
+  const int2 run = load_runs(runs, rs, re, 0, lane);
+  const int32_t len = rs + lane < re ? run.y : 0;
+  const int32_t incl = wave_incl_scan(len);
+  const int32_t total = readlane(incl, kWave - 1);
+  if (total == 0) return;
+  lk->base[lane] = run.x - (incl - len);
+  int32_t carry = 0;
+  const int32_t s = pairs[item_index(lk, len, incl - len, total, 0, &carry, lane)].x;
+  int32_t fresh = 0;
+  for (uint64_t m = ballot(lane < total && s != row); m != 0; ++fresh) {
+    m &= ~ballot(s == readlane(s, __builtin_ctzll(m)));
+  }
+  if (lane == 0) {
+    // The other blocks of a long row hold about as many; a hub row counts as
+    // 2^20 items at most.
+    const int64_t items = static_cast<int64_t>(total) * ((re - rs + kWave - 1) / kWave);
+    const uint32_t w = static_cast<uint32_t>(items < (1 << 20) ? items : (1 << 20));
+    atomicAdd(&weight[0], w);
+    if (evicts_soon(fresh, total, capacity)) atomicAdd(&weight[1], w);
+  }
+}
+
+// The rows are counted unless most of the sampled items are in rows that evict.
+// Power-law graphs: cg 0.99, chunks of 20,000 of 600,000 rows 0.87 at capacity
+// 512 (152 ms counted, 124 not), chunks of 5,000 of 2.4 M rows 0.52 (252 and
+// 217); 0.71 for chunks of 8,192 of them at capacity 64, where counting is
+// ahead by 1 to 2 % (130 and 132).
+__device__ __forceinline__ bool sample_counts(const uint32_t *__restrict__ weight) {
+  return 2 * weight[1] <= weight[0]; // weights are at most 2^28
+}
+
 // Registers: with counting, up to capacity 128 at most 64, so that 8 waves
 // share a SIMD, and two fit beside the four of a tier-2 workgroup; without it
 // the kernel needs 33 to 62 by itself.
@@ -307,7 +360,9 @@ template <int CELLS, bool COUNT> constexpr int ovf_min_waves() {
 
 // WIDE: chunks of more than 2^12 rows, whose candidates need a whole word in
 // the counting table.  COUNT: rows are counted (sample_shared in csg_local.hip);
-// false feeds every item to the sketch.
+// false feeds every item to the sketch.  `sampled`, when given: the sums of
+// ovf_sample_kernel; both forms are launched and the one that they rule out
+// ends at once.
 template <int CELLS, bool WIDE, bool COUNT>
 __global__ void __launch_bounds__(kOvfBlock, (ovf_min_waves<CELLS, COUNT>()))
     ovf_sketch_kernel(int32_t n, int32_t k, int32_t chunk_size,
@@ -315,7 +370,9 @@ __global__ void __launch_bounds__(kOvfBlock, (ovf_min_waves<CELLS, COUNT>()))
                       const int2 *__restrict__ pairs, uint64_t *__restrict__ table,
                       const int32_t *__restrict__ list,
                       const int32_t *__restrict__ list_count, uint32_t *__restrict__ claim,
-                      int32_t *__restrict__ row_valid, int64_t l0, int64_t l1) {
+                      int32_t *__restrict__ row_valid, const uint32_t *__restrict__ sampled,
+                      int64_t l0, int64_t l1) {
+  if (sampled != nullptr && sample_counts(sampled) != COUNT) return;
   __shared__ RunLookup s_lookup[kOvfWaves];
   RowStream<CELLS, WIDE, COUNT> st;
   __shared__ uint32_t s_count[kOvfWaves][COUNT ? decltype(st.counter)::kWords : 1];
@@ -461,8 +518,8 @@ template <int CELLS>
 void launch_ovf_sketch(Context &ctx, int32_t n, int32_t k, int32_t chunk_size,
                        const int32_t *d_ptr, const int2 *runs, const int2 *pairs,
                        uint64_t *d_table, const int32_t *list, const int32_t *list_count,
-                       uint32_t *claim, int32_t *d_row_valid, int64_t l0, int64_t l1,
-                       int64_t rows, bool count) {
+                       uint32_t *claim, int32_t *d_row_valid, const uint32_t *sampled, int64_t l0,
+                       int64_t l1, int64_t rows, bool count) {
   // A wave per row at most: rows = the launch's row slots when the host knows
   // them (a grid sized for every row of the matrix made a one-chunk launch
   // dispatch thousands of workgroups that found no row, holding back the
@@ -471,12 +528,11 @@ void launch_ovf_sketch(Context &ctx, int32_t n, int32_t k, int32_t chunk_size,
   // the finite-element matrix 4.0 -> 4.3 ms, cg of the geometric graph 1.3 ->
   // 1.6).
   const int g = ctx.grid_for(ceil_div64(rows >= 0 ? rows : n, kOvfWaves), kOvfBlock, 1);
-  fill_u32(ctx, claim, kClaimWords, 0u);
   auto *kernel = !count ? ovf_sketch_kernel<CELLS, false, false>
                  : chunk_size <= 4096 ? ovf_sketch_kernel<CELLS, false, true>
                                       : ovf_sketch_kernel<CELLS, true, true>;
   kernel<<<g, kOvfBlock, 0, ctx.stream>>>(n, k, chunk_size, d_ptr, runs, pairs, d_table, list,
-                                          list_count, claim, d_row_valid, l0, l1);
+                                          list_count, claim, d_row_valid, sampled, l0, l1);
   SP_LAUNCH_CHECK();
 }
 
@@ -506,7 +562,7 @@ void chunk_sketch_top_k(Context &ctx, int32_t n, int32_t nnz, int32_t k, int32_t
                         const int32_t *d_col_ptr, const int32_t *d_row_ind,
                         uint64_t *d_table, const int32_t *d_chunks,
                         const int32_t *d_chunk_count, hipEvent_t prepared,
-                        int32_t *d_row_valid, int64_t host_list_len, bool count) {
+                        int32_t *d_row_valid, int64_t host_list_len, CountRows count) {
   SP_EXPECT(k <= 512, "k must be <= 512");
   SP_EXPECT(m_capacity % 32 == 0 && m_capacity >= 32 && m_capacity <= 512,
             "sketch capacity must be a multiple of 32 in [32, 512]");
@@ -532,7 +588,8 @@ void chunk_sketch_top_k(Context &ctx, int32_t n, int32_t nnz, int32_t k, int32_t
                                                        d_chunk_count, task_off, runs, l0, l1);
     SP_LAUNCH_CHECK();
   };
-  auto sketch_launch = [&](uint32_t *cl, int64_t l0, int64_t l1) {
+  auto sketch_form = [&](uint32_t *cl, const uint32_t *sampled, int64_t l0, int64_t l1,
+                         bool counted) {
     // Row slots of list entries [l0, l1) when the list's length is known.
     int64_t rows = -1;
     if (d_chunks == nullptr) {
@@ -545,7 +602,7 @@ void chunk_sketch_top_k(Context &ctx, int32_t n, int32_t nnz, int32_t k, int32_t
 #define SP_CASE(C)                                                                         \
   case C:                                                                                  \
     launch_ovf_sketch<C>(ctx, n, k, chunk_size, d_ptr, runs, pairs, d_table, d_chunks,     \
-                         d_chunk_count, cl, d_row_valid, l0, l1, rows, count);             \
+                         d_chunk_count, cl, d_row_valid, sampled, l0, l1, rows, counted);  \
     break;
       SP_CASE(1) SP_CASE(2) SP_CASE(3) SP_CASE(4) SP_CASE(5) SP_CASE(6)
       SP_CASE(7) SP_CASE(8) SP_CASE(9) SP_CASE(10) SP_CASE(11) SP_CASE(12)
@@ -555,7 +612,25 @@ void chunk_sketch_top_k(Context &ctx, int32_t n, int32_t nnz, int32_t k, int32_t
       break;
     }
   };
-  if (d_chunks == nullptr || host_list_len < 2) {
+  auto sketch_launch = [&](uint32_t *cl, int64_t l0, int64_t l1) {
+    fill_u32(ctx, cl, kClaimWords, 0u);
+    sketch_form(cl, nullptr, l0, l1, count == CountRows::kYes);
+  };
+  if (count == CountRows::kSampled) {
+    SP_EXPECT(d_chunks == nullptr, "internal: listed chunks come with a classification");
+    runs_launch(0, -1);
+    if (prepared != nullptr) SP_HIP(hipEventRecord(prepared, ctx.stream));
+    // One form claims rows, so the second set of counters is free.
+    uint32_t *weight = claim + kClaimWords;
+    fill_u32(ctx, claim, kClaimWords + 2, 0u);
+    ovf_sample_kernel<<<kSampleRows / kOvfWaves, kOvfBlock, 0, ctx.stream>>>(
+        n, m_capacity, d_ptr, runs, pairs, weight);
+    SP_LAUNCH_CHECK();
+    sketch_form(claim, weight, 0, -1, true);
+    sketch_form(claim, weight, 0, -1, false);
+    return;
+  }
+  if (host_list_len < 2) {
     runs_launch(0, -1);
     if (prepared != nullptr) SP_HIP(hipEventRecord(prepared, ctx.stream));
     sketch_launch(claim, 0, -1);

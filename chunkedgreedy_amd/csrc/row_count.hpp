@@ -30,6 +30,13 @@ constexpr int row_table_entries(int M) {
   return h;
 }
 
+// Whether a row's stream will likely need evictions, from its first batch:
+// nearly all of the batch were new candidates (`fresh` of them) and the block's
+// `total` items are more than twice the capacity M.
+__device__ __forceinline__ bool evicts_soon(int32_t fresh, int32_t total, int32_t M) {
+  return fresh > kWave - 8 && total > 2 * M;
+}
+
 // One wave's counter.  H: table entries.  WIDE: candidates are any row index
 // and the table has a second word per entry; otherwise they are below 2^12
 // (chunk-local) and an entry is one word, (candidate 12 bits | field 10 bits |
@@ -151,13 +158,11 @@ template <int CELLS, int H, bool WIDE> struct RowCounter {
     return true;
   }
 
-  // After a row's first batch: whether its stream, whose next `total` items
-  // include that batch, will likely need evictions.  Nearly all of the batch
-  // were new candidates and twice the capacity follows: on power-law rows
-  // (about 250 items over 1,000 candidates) counting the first 128 and
-  // turning them into slots cost more than it saved, csg 18.9 -> 19.4 ms.
+  // After a row's first batch: evicts_soon.  On power-law rows (about 250 items
+  // over 1,000 candidates) counting the first 128 and turning them into slots
+  // cost more than it saved, csg 18.9 -> 19.4 ms.
   __device__ __forceinline__ bool will_evict(int32_t total) const {
-    return filled > kWave - 8 && total > 2 * M;
+    return evicts_soon(filled, total, M);
   }
 
   // Slot q * 64 + lane's row (-1: empty) and weight in each lane, from the
