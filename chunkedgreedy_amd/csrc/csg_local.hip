@@ -617,7 +617,7 @@ __global__ void __launch_bounds__(kLocalThreads)
           f0 = 0;
           open_block(pb, re);
         }
-        store.select_top_k(k, out);
+        store.template select_top_k<true>(k, out);
       }
       if (row_valid != nullptr && lane == 0) row_valid[row] = min(k, store.filled);
     }

@@ -268,7 +268,8 @@ template <int CELLS, bool WIDE, bool COUNT> struct RowStream {
         return;
       }
     }
-    store.select_top_k(k, out);
+    // Not counted: rows that evict, full at the end, or that hold hardly an item.
+    store.template select_top_k<COUNT>(k, out);
   }
 };
 
@@ -304,8 +305,10 @@ __device__ __forceinline__ void feed_block(Stream &st, RunLookup *lk,
 // weight[0] is the sum of their items, weight[1] of those in rows that will
 // likely evict (evicts_soon).  Rows that evict all along gain nothing from
 // counting and pay for its table and registers: cg of a power-law graph of
-// 150,000 rows, capacity 512: 264 ms counted, 217 not; chunks of 20,000 rows of
-// one of 600,000: 152 and 124.  That neighbouring rows share no columns
+// 150,000 rows, capacity 512: 262 ms counted, 210 not; chunks of 20,000 rows of
+// one of 600,000: 153 and 121.  (Rows that evict late would gain still: cg of
+// the finite-element matrix, 2,100 items over 375 candidates a row, capacity
+// 320: 40.7 ms counted, 43.2 not.)  That neighbouring rows share no columns
 // (sample_shared) does not tell here, where a row meets the whole matrix:
 // scrambled blocks of 64 rows, 600,000 rows of 14, capacity 256: 5.5 ms
 // counted, 8.9 not.
@@ -344,7 +347,7 @@ __global__ void __launch_bounds__(kOvfBlock)
 
 // The rows are counted unless most of the sampled items are in rows that evict.
 // Power-law graphs: cg 0.99, chunks of 20,000 of 600,000 rows 0.87 at capacity
-// 512 (152 ms counted, 124 not), chunks of 5,000 of 2.4 M rows 0.52 (252 and
+// 512 (153 ms counted, 121 not), chunks of 5,000 of 2.4 M rows 0.52 (252 and
 // 217); 0.71 for chunks of 8,192 of them at capacity 64, where counting is
 // ahead by 1 to 2 % (130 and 132).
 __device__ __forceinline__ bool sample_counts(const uint32_t *__restrict__ weight) {

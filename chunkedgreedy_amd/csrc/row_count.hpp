@@ -288,7 +288,7 @@ template <int CELLS, int H, bool WIDE> struct RowCounter {
       }
       wave_lds_order();
       empty();
-      store.emit_lists(k, out, fk, fw);
+      store.template emit_lists<true>(k, out, fk, fw);
     }
   }
 };

@@ -504,8 +504,9 @@ template <int CELLS> struct WaveSketch {
   // Reference select_top_k: per-logical-lane selection sort (strict '>',
   // stop at -1), then up to k rounds emitting the head of the lane with the
   // largest head weight (ties -> smaller lane; exhausted lanes show 0.0f).
-  // Writes all k entries of `out` (unused ones as the zero entry).
-  __device__ __forceinline__ void select_top_k(int32_t k, uint64_t *out) {
+  // Writes all k entries of `out` (unused ones as the zero entry).  NETWORK: see
+  // emit_lists.
+  template <bool NETWORK> __device__ __forceinline__ void select_top_k(int32_t k, uint64_t *out) {
     if constexpr (CELLS <= 2) {
       select_top_k_sorted(k, out);
       return;
@@ -525,14 +526,36 @@ template <int CELLS> struct WaveSketch {
         fw[2 * j + 1] = hw;
       }
     }
-    emit_lists(k, out, fk, fw);
+    emit_lists<NETWORK>(k, out, fk, fw);
   }
 
+  // Up to this many live entries are merged rather than sorted (emit_lists).
+  static constexpr int kFewEntries = 12;
+
   // select_top_k from the cells of logical lane L in physical lane L (< 32;
-  // the upper half's values are not used).
-  __device__ __forceinline__ void emit_lists(int32_t k, uint64_t *out, int32_t (&fk)[CELLS],
-                                             float (&fw)[CELLS]) {
+  // the upper half's values are not used).  NETWORK: past four cells, rows of
+  // up to 128 live entries take the sorting network.  Kernels whose rows are
+  // either full or empty leave it out: beside the merge it costs 26 to 104
+  // spilled scalar registers, and the lists, changed through the reference,
+  // stay in scratch memory (cg of a power-law graph of 150,000 rows, capacity
+  // 512: 217 ms with both, 212 without).  Where the network is in, the lists
+  // are better left there: copied, they push other values into scratch (csg of
+  // the finite-element matrix 4.00 -> 4.33 ms).
+  template <bool NETWORK>
+  __device__ __forceinline__ void emit_lists(int32_t k, uint64_t *out, int32_t (&keys)[CELLS],
+                                             float (&weights)[CELLS]) {
     const int lane = lane_id();
+    int32_t own_keys[CELLS];
+    float own_weights[CELLS];
+    if constexpr (!NETWORK) {
+#pragma unroll
+      for (int c = 0; c < CELLS; ++c) {
+        own_keys[c] = keys[c];
+        own_weights[c] = weights[c];
+      }
+    }
+    int32_t (&fk)[CELLS] = NETWORK ? keys : own_keys;
+    float (&fw)[CELLS] = NETWORK ? weights : own_weights;
     // Selection sort, literally as the reference (not stable).
 #pragma unroll
     for (int i = 0; i < CELLS - 1; ++i) {
@@ -562,11 +585,16 @@ template <int CELLS> struct WaveSketch {
         }
       }
     }
-    // Up to 128 live entries: one sorting network.  The merge below costs
-    // about 45 wave instructions per emitted entry (k = 77 at CELLS = 10: some
-    // 3,500 a row, more than the row's counting; the network about 700).
-    if constexpr (CELLS >= 3) {
-      if (CELLS <= 4 || filled <= 128) {
+    // Up to 128 live entries: one sorting network, about 700 wave instructions.
+    // The merge below costs about 45 per emitted entry (k = 77 at CELLS = 10:
+    // some 3,500 a row, more than the row's counting), which is less for a few
+    // entries (csg of scrambled blocks of 600,000 rows, capacity 512: 446 ->
+    // 402 us).
+    if constexpr (CELLS >= 3 && CELLS <= 4) {
+      emit_sorted_lists(k, out, fk, fw);
+      return;
+    } else if constexpr (NETWORK && CELLS > 4) {
+      if (filled > kFewEntries && filled <= 128) {
         emit_sorted_lists(k, out, fk, fw);
         return;
       }
