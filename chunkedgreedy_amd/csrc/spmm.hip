@@ -46,6 +46,12 @@ constexpr int kSpmmDepth = 8; // B rows in flight per row group
 constexpr int kLongRow = SPORDER_SPMM_LONG_ROW;
 constexpr int kSegLen = SPORDER_SPMM_SEGMENT;
 constexpr int kTileRows = kSpmmTileRows; // rows of a tile of an SpMM plan
+// Ragged widths up to 32 columns: from this many rows on (a wave of 64 rows for
+// every wave the device holds) the groups of a wave claim its rows, below it
+// each group has its own, at least 8 lanes a row.  Claiming, in us, against its
+// own row: 10,000 rows of 60, N = 30 111 and 45; 200,000 rows of 10, N = 1 55
+// and 45; power-law rows, 600,000 of 12, N = 30 350 and 400.
+constexpr int kClaimedRows = 1 << 19;
 
 // Long rows: rows past kLongRow nonzeros leave the row-split launch, which
 // appends a descriptor; each becomes nseg segment units whose partials the
@@ -804,7 +810,8 @@ void launch_rowsplit_gs(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr
   // wider rows the fixed assignment keeps more waves in flight.  With a tile
   // list only the listed tiles' rows are computed.
   const int64_t waves = tiles == nullptr ? ceil_div64(n, rpw) : ntiles * (kTileRows / rpw);
-  if (G <= 8 && N <= V * G) {
+  const bool ragged = RG || V == 1;
+  if (G <= 8 && N <= V * G && !(ragged && n < kClaimedRows)) {
     const int64_t dyn_waves = tiles == nullptr ? ceil_div64(n, kWave) : ntiles;
     const int64_t blocks = ceil_div64(dyn_waves, kSpmmWaves);
     spmm_rows_dyn<G, CS, V, RG><<<dim3(static_cast<unsigned>(blocks)), kSpmmBlock, 0, ctx.stream>>>(
@@ -884,7 +891,8 @@ void spmm_rowsplit(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr,
                             ntiles, sc);
     return;
   }
-  const int32_t q = (N + 3) / 4; // float4 column slices
+  int32_t q = (N + 3) / 4; // float4 column slices
+  if (q < 8 && n < kClaimedRows && is_ragged(N, B, C)) q = 8; // 8 lanes a row
   if (q <= 1) {
     launch_rowsplit_g<1>(ctx, n, nnz, ptr, ind, val, N, B, C, w, seg_cap, long_cap,
                           tiles, ntiles, sc);

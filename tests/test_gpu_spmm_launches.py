@@ -1,0 +1,39 @@
+"""What a ragged SpMM call launches, from the kernels that ran: few rows are
+spread over the chip, and small calls are not mostly launches."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def kernels(call):
+    """Names of the library's kernels that `call` runs, in order."""
+    call()
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU,
+                                            torch.profiler.ProfilerActivity.CUDA]) as prof:
+        call()
+        torch.cuda.synchronize()
+    return [e.name for e in prof.events() if "sporder_hip" in e.name]
+
+
+def case(n, deg, N, seed=5):
+    """A uniform matrix on the GPU (ptr, ind, val), B and an output."""
+    rng = np.random.default_rng(seed)
+    keys = np.unique(np.repeat(np.arange(n), deg) * n + rng.integers(0, n, n * deg))
+    ptr = np.concatenate([[0], np.cumsum(np.bincount(keys // n, minlength=n))])
+    p, i = (torch.from_numpy(a.astype(np.int32)).to("cuda:0") for a in (ptr, keys % n))
+    v = torch.ones(i.numel(), device="cuda:0")
+    return p, i, v, torch.ones((n, N), device="cuda:0"), torch.empty((n, N), device="cuda:0")
+
+
+@pytest.mark.parametrize("N", [1, 3, 7, 30])
+def test_few_rows_have_groups_of_their_own(sporder, N):
+    """300,000 rows, 64 to a wave, would fill little more than half of the chip."""
+    print(f"[spmm_launches] own groups N={N}", flush=True)
+    p, i, v, B, out = case(300_000, 3, N)
+    names = kernels(lambda: sporder.spmm_csr(p, i, v, B, out=out))
+    assert any("spmm_rowsplit_v4<8" in k for k in names)
+    assert not any("spmm_rows_dyn" in k for k in names)
