@@ -489,6 +489,99 @@ __global__ void __launch_bounds__(kSpmmBlock)
   }
 }
 
+// Small calls of ragged widths in one launch, a row per group of G lanes; a
+// workgroup's rows past kLongRow are then done by all of its groups, a segment
+// each, the partial rows added in LDS in the stated order.  What bounds it is
+// the launch and three dependent loads: 2,000 rows of 8, N = 30: 26.4 us a call
+// (fill, rows, segments and fix-up launched one after another: 32.4).
+template <int BLOCK, int G, bool CS, int V, bool RG>
+__global__ void __launch_bounds__(BLOCK)
+    spmm_rows_small(int32_t n, const int32_t *__restrict__ ptr, const int32_t *__restrict__ ind,
+                    const float *__restrict__ val, int32_t N, const float *__restrict__ B,
+                    float *__restrict__ C, const float *__restrict__ rs,
+                    const float *__restrict__ cs) {
+  constexpr int R = BLOCK / G;
+  typedef typename ColsOf<V>::T T;
+  __shared__ T s_part[R][G];
+  __shared__ T s_carry[2][G]; // a row's sum so far when its segments pass a round
+  __shared__ int32_t s_long[R], s_first[R + 1], s_count;
+  const int gl = lane_id() % G, gbase = lane_id() - gl;
+  const int32_t gid = threadIdx.x / G;
+  if (threadIdx.x == 0) s_count = 0;
+  __syncthreads();
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * R + gid;
+  const bool row_ok = row < n;
+  const int32_t s = row_ok ? ptr[row] : 0;
+  int32_t e = row_ok ? ptr[row + 1] : 0;
+  const bool is_long = e - s > kLongRow;
+  if (is_long) {
+    if (gl == 0) s_long[atomicAdd(&s_count, 1)] = static_cast<int32_t>(row);
+    e = s;
+  }
+  for (int32_t cb = 0; cb < N; cb += G * V) {
+    const int32_t at = cb + gl * V;
+    const bool col_ok = at < N;
+    const int32_t col0 = slice_col<V, RG>(at, N);
+    const T acc = group_dot<G, CS, V, RG>(s, e, ind, val, N, col0, col_ok, B, gl, gbase, cs);
+    if (row_ok && col_ok && !is_long) {
+      store_nt<RG>(C + row * N + col0, row_scaled(rs, row, acc), RG ? at - col0 : 0);
+    }
+  }
+  __syncthreads();
+  const int32_t count = s_count;
+  if (count == 0) return; // the whole workgroup
+  // s_first[i]: the first unit (segment) of the i-th long row.
+  if (threadIdx.x == 0) {
+    int32_t units = 0;
+    for (int32_t i = 0; i < count; ++i) {
+      s_first[i] = units;
+      units += (ptr[s_long[i] + 1] - ptr[s_long[i]] + kSegLen - 1) / kSegLen;
+    }
+    s_first[count] = units;
+  }
+  __syncthreads();
+  const int32_t units = s_first[count];
+  for (int32_t cb = 0; cb < N; cb += G * V) {
+    const int32_t at = cb + gl * V;
+    const bool col_ok = at < N;
+    const int32_t col0 = slice_col<V, RG>(at, N);
+    int parity = 0;
+    for (int32_t u0 = 0; u0 < units; u0 += R, parity ^= 1) {
+      const int32_t u = u0 + gid;
+      const bool ok = u < units;
+      int32_t i = 0; // the long row of unit u: the last one with s_first[i] <= u
+      for (int32_t hi = count - 1; ok && i < hi;) {
+        const int32_t mid = (i + hi + 1) / 2;
+        if (s_first[mid] <= u) {
+          i = mid;
+        } else {
+          hi = mid - 1;
+        }
+      }
+      const int32_t lr = s_long[i], seg = u - s_first[i];
+      const int32_t us = ok ? ptr[lr] + seg * kSegLen : 0, re = ok ? ptr[lr + 1] : 0;
+      const int32_t ue = re - us < kSegLen ? re : us + kSegLen;
+      s_part[gid][gl] = group_dot<G, CS, V, RG>(us, ue, ind, val, N, col0, col_ok, B, gl, gbase, cs);
+      __syncthreads();
+      // The group of the row's first unit in this round adds its units up.
+      if (ok && (seg == 0 || gid == 0)) {
+        const int32_t end = s_first[i + 1];
+        const int32_t m = (end < u0 + R ? end : u0 + R) - u;
+        T sum = s_part[gid][gl];
+        if (seg != 0) sum = added(s_carry[parity][gl], sum);
+        for (int32_t q = 1; q < m; ++q) sum = added(sum, s_part[gid + q][gl]);
+        if (end > u0 + R) {
+          s_carry[parity ^ 1][gl] = sum;
+        } else if (col_ok) {
+          store_nt<RG>(C + static_cast<int64_t>(lr) * N + col0, row_scaled(rs, lr, sum),
+                       RG ? at - col0 : 0);
+        }
+      }
+      __syncthreads();
+    }
+  }
+}
+
 // One wave per row, lanes over columns, one gather in flight, same stated
 // order (long rows as segment chains added left to right) with no scratch: the
 // no-allocation entry's way for widths that are not a multiple of 4 whose long
@@ -862,6 +955,61 @@ void launch_rowsplit_g(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr,
   }
 }
 
+// Lanes per row of spmm_rows_small: at least 8, so that a row's nonzeros are
+// loaded 8 at a time however narrow B is.
+int small_group(int32_t N) {
+  const int32_t q = (N + 3) / 4;
+  return q <= 8 ? 8 : q <= 16 ? 16 : q <= 32 ? 32 : 64;
+}
+
+// Ragged calls that spmm_rows_small takes.  Where a call is mostly launches it
+// saves three of four (in us, against the other launches; 40,000 rows of 10):
+// N = 1 30 and 35, N = 30 36 and 39, N = 47 39 and 42; past 128 columns it has
+// few rows in a workgroup (N = 150: 73 and 69), and on larger matrices its long
+// rows keep to one CU (power-law, 100,000 rows, N = 30: 245 and 202).
+bool is_small(int32_t nnz, int32_t N, const float *B, const float *C) {
+  return is_ragged(N, B, C) && nnz <= (1 << (small_group(N) == 64 ? 18 : 19));
+}
+
+template <int G, int V, bool RG>
+void launch_small_g(Context &ctx, int32_t n, const int32_t *ptr, const int32_t *ind,
+                    const float *val, int32_t N, const float *B, float *C, const SpmmScale &sc) {
+  // The larger workgroup has more groups for a long row; where it leaves CUs
+  // without one, rows of a few hundred nonzeros are better spread.
+  const bool wide = ceil_div64(n, 1024 / G) >= ctx.num_cus;
+  const int block = wide ? 1024 : 256;
+  const dim3 grid(static_cast<unsigned>(ceil_div64(n, block / G)));
+  auto *kernel = sc.col != nullptr
+                     ? (wide ? spmm_rows_small<1024, G, true, V, RG> : spmm_rows_small<256, G, true, V, RG>)
+                     : (wide ? spmm_rows_small<1024, G, false, V, RG>
+                             : spmm_rows_small<256, G, false, V, RG>);
+  kernel<<<grid, block, 0, ctx.stream>>>(n, ptr, ind, val, N, B, C, sc.row, sc.col);
+  SP_LAUNCH_CHECK();
+}
+
+void launch_small(Context &ctx, int32_t n, const int32_t *ptr, const int32_t *ind,
+                  const float *val, int32_t N, const float *B, float *C,
+                  const SpmmScale &sc = SpmmScale{}) {
+  if (N < 4) {
+    launch_small_g<8, 1, false>(ctx, n, ptr, ind, val, N, B, C, sc);
+    return;
+  }
+  switch (small_group(N)) {
+  case 8:
+    launch_small_g<8, 4, true>(ctx, n, ptr, ind, val, N, B, C, sc);
+    break;
+  case 16:
+    launch_small_g<16, 4, true>(ctx, n, ptr, ind, val, N, B, C, sc);
+    break;
+  case 32:
+    launch_small_g<32, 4, true>(ctx, n, ptr, ind, val, N, B, C, sc);
+    break;
+  default:
+    launch_small_g<64, 4, true>(ctx, n, ptr, ind, val, N, B, C, sc);
+    break;
+  }
+}
+
 } // namespace
 
 size_t spmm_ws_bytes(int32_t nnz, int32_t N) {
@@ -880,6 +1028,10 @@ void spmm_rowsplit(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr,
                    const SpmmScale &sc = SpmmScale{}) {
   if (seg_cap < 0) seg_cap = max_segments(nnz);
   if (long_cap < 0) long_cap = max_long_rows(nnz);
+  if (tiles == nullptr && is_small(nnz, N, B, C) && w.ctl != nullptr) {
+    launch_small(ctx, n, ptr, ind, val, N, B, C, sc);
+    return;
+  }
   // Every width and alignment takes the row groups, long rows in segments.
   // The one-wave-per-row kernel that ragged widths took before has one gather
   // in flight and walks a long row alone: N = 47 on a power-law graph of

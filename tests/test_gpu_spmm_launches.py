@@ -37,3 +37,15 @@ def test_few_rows_have_groups_of_their_own(sporder, N):
     names = kernels(lambda: sporder.spmm_csr(p, i, v, B, out=out))
     assert any("spmm_rowsplit_v4<8" in k for k in names)
     assert not any("spmm_rows_dyn" in k for k in names)
+
+
+@pytest.mark.parametrize("N", [2, 7, 47, 150])
+@pytest.mark.parametrize("how", ["row_split", "scaled"])
+def test_small_calls_are_one_launch(sporder, how, N):
+    print(f"[spmm_launches] {how} N={N}", flush=True)
+    p, i, v, B, out = case(2_000, 8, N)
+    scale = torch.ones(2_000, device="cuda:0")
+    calls = {"row_split": lambda: sporder.spmm_csr(p, i, v, B, out=out),
+             "scaled": lambda: sporder.spmm_csr_scaled(p, i, v, B, row_scale=scale, out=out)}
+    names = kernels(calls[how])
+    assert len(names) == 1 and "spmm_rows_small" in names[0]

@@ -15,18 +15,66 @@ DEV = "cuda:0"
 N_ROWS = 1111
 
 
-@pytest.fixture(scope="module")
-def matrix():
-    """Rows of 0..80 nonzeros, and five around and past the 512-nonzero
-    segments (511, 512, 513, 1025, 1100)."""
-    rng = np.random.default_rng(21)
-    lens = rng.integers(0, 81, N_ROWS)
-    lens[[5, 64, 300, 777, N_ROWS - 1]] = [511, 512, 513, 1025, 1100]
-    lens[[0, 63, 128]] = 0
-    ind = np.concatenate([np.sort(rng.choice(N_ROWS, k, replace=False)) for k in lens])
+def from_lengths(n, lens, seed):
+    """Rows of the given lengths, columns drawn with repetition when a row is
+    longer than n."""
+    rng = np.random.default_rng(seed)
+    ind = np.concatenate([np.sort(rng.choice(n, k, replace=k > n)) for k in lens])
     ptr = np.concatenate([[0], np.cumsum(lens)])
     val = rng.uniform(-1, 1, ind.size).astype(np.float32)
     return ptr.astype(np.int32), ind.astype(np.int32), val
+
+
+def mixed(n, most, seed=21):
+    """Rows of 0..most nonzeros, and five around and past the 512-nonzero
+    segments (511, 512, 513, 1025, 1100)."""
+    lens = np.random.default_rng(seed).integers(0, most + 1, n)
+    lens[[5, 64, 300, 777, n - 1]] = [511, 512, 513, 1025, 1100]
+    lens[[0, 63, 128]] = 0
+    return from_lengths(n, lens, seed)
+
+
+def mostly_long():
+    """Neighbouring rows past a segment, and rows of 20,000 and 70,000
+    nonzeros: more segments than a workgroup has row groups."""
+    rng = np.random.default_rng(22)
+    lens = rng.integers(0, 30, 700)
+    lens[200:300] = rng.integers(500, 1400, 100)
+    lens[[3, 250]] = [20_000, 70_000]
+    return from_lengths(700, lens, 22)
+
+
+def many_rows():
+    """2^19 and some rows of 0..4 nonzeros, and the long rows of `mixed`."""
+    n = (1 << 19) + 77
+    lens = np.random.default_rng(23).integers(0, 5, n)
+    lens[[5, 64, 300, 777, n - 1]] = [511, 512, 513, 1025, 1100]
+    rows = np.repeat(np.arange(n), lens)
+    rng = np.random.default_rng(24)
+    ind = rng.integers(0, n, rows.size)
+    ind = ind[np.lexsort((ind, rows))]
+    return (np.concatenate([[0], np.cumsum(lens)]).astype(np.int32), ind.astype(np.int32),
+            rng.uniform(-1, 1, ind.size).astype(np.float32))
+
+
+# One launch (ragged widths up to 2^19 nonzeros, 2^18 past 128 columns), the
+# launches of a larger matrix, and one launch with more segments than groups.
+MATRICES = {"small": lambda: mixed(N_ROWS, 80), "large": lambda: mixed(4 * N_ROWS, 260),
+            "long": mostly_long}
+
+
+@pytest.fixture(scope="module", params=sorted(MATRICES))
+def matrix(request):
+    m = MATRICES[request.param]()
+    assert (m[1].size > 1 << 19) == (request.param == "large")
+    assert m[1].size > 1 << 19 or m[1].size <= 1 << 18
+    return m
+
+
+@pytest.fixture(scope="module")
+def rows_to_claim():
+    """More rows than have a group of their own: claimed up to 32 columns."""
+    return many_rows()
 
 
 def shifted(a, words):
@@ -41,14 +89,25 @@ def shifted(a, words):
 @pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 7, 13, 16, 17, 31, 33, 47, 64, 67, 127, 130, 259])
 @pytest.mark.parametrize("words", [0, 1, 2, 3])
 def test_spmm_widths_and_alignments(matrix, N, words):
+    check_all_calls(matrix, N, words)
+
+
+@pytest.mark.parametrize("N,words", [(1, 0), (2, 3), (3, 1), (4, 1), (5, 0), (7, 2), (13, 0),
+                                     (16, 3), (31, 0), (32, 2)])
+def test_spmm_claimed_rows(rows_to_claim, N, words):
+    check_all_calls(rows_to_claim, N, words)
+
+
+def check_all_calls(matrix, N, words):
     from chunkedgreedy_amd import sporder
 
     ptr, ind, val = matrix
     rng = np.random.default_rng(N)
-    Bh = rng.standard_normal((N_ROWS, N)).astype(np.float32)
-    rs, cs = (rng.uniform(0.05, 2.0, N_ROWS).astype(np.float32) for _ in range(2))
+    n = ptr.size - 1
+    Bh = rng.standard_normal((n, N)).astype(np.float32)
+    rs, cs = (rng.uniform(0.05, 2.0, n).astype(np.float32) for _ in range(2))
     want = oracle.spmm_csr(ptr, ind, val, Bh)
-    p, i, v = (torch.from_numpy(x).to(DEV) for x in matrix)
+    p, i, v = (torch.from_numpy(x).to(DEV) for x in (ptr, ind, val))
     _, B = shifted(Bh, words)
     buf, out = shifted(np.zeros_like(Bh), words)
     plan = sporder.spmm_plan(p, i)
