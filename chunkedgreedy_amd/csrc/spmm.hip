@@ -1238,16 +1238,26 @@ int32_t sporder_spmm_csr_noalloc(sporder_context_t h, int32_t n, int32_t nnz,
   Context &ctx = h->impl;
   char *base = static_cast<char *>(noalloc_scratch(ctx.device));
   std::lock_guard<std::mutex> call_lock(noalloc_call_mu[ctx.device]);
-  // Exact need: count the long rows and their segments first.
+  if (is_small(nnz, cols, d_b, d_c)) { // no scratch
+    launch_small(ctx, n, d_ptr, d_ind, d_val, cols, d_b, d_c);
+    ctx.sync();
+    return 0;
+  }
   LongCtl *ctl = reinterpret_cast<LongCtl *>(base);
-  fill_u32(ctx, ctl, sizeof(LongCtl) / 4, 0u);
-  const int gc = ctx.grid_for(ceil_div64(n, 256), 256, 2);
-  spmm_count_long<<<gc, 256, 0, ctx.stream>>>(n, d_ptr, ctl);
-  SP_LAUNCH_CHECK();
-  SP_HIP(hipMemcpyAsync(ctx.host_words, ctl, sizeof(LongCtl), hipMemcpyDeviceToHost,
-                        ctx.stream));
-  ctx.sync();
-  const int64_t long_rows = ctx.host_words[0], segments = ctx.host_words[1];
+  int64_t long_rows = max_long_rows(nnz), segments = max_segments(nnz);
+  if (spmm_ws_bytes(nnz, cols) > kNoAllocBytes) {
+    // What nnz nonzeros can need at most does not fit (otherwise the readback,
+    // some 14 us, is left out): count the long rows and their segments.
+    fill_u32(ctx, ctl, sizeof(LongCtl) / 4, 0u);
+    const int gc = ctx.grid_for(ceil_div64(n, 256), 256, 2);
+    spmm_count_long<<<gc, 256, 0, ctx.stream>>>(n, d_ptr, ctl);
+    SP_LAUNCH_CHECK();
+    SP_HIP(hipMemcpyAsync(ctx.host_words, ctl, sizeof(LongCtl), hipMemcpyDeviceToHost,
+                          ctx.stream));
+    ctx.sync();
+    long_rows = ctx.host_words[0];
+    segments = ctx.host_words[1];
+  }
   const size_t need = ws_bytes<LongCtl>(1) + ws_bytes<LongRow>(static_cast<size_t>(long_rows)) +
                       ws_bytes<int32_t>(static_cast<size_t>(segments)) +
                       ws_bytes<float>(static_cast<size_t>(segments) * cols);

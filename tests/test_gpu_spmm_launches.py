@@ -49,3 +49,14 @@ def test_small_calls_are_one_launch(sporder, how, N):
              "scaled": lambda: sporder.spmm_csr_scaled(p, i, v, B, row_scale=scale, out=out)}
     names = kernels(calls[how])
     assert len(names) == 1 and "spmm_rows_small" in names[0]
+
+
+@pytest.mark.parametrize("n,deg,N,most", [(2_000, 8, 30, 1), (2_000, 8, 47, 1),
+                                          (70_000, 10, 3, 4), (70_000, 10, 47, 4)])
+def test_noalloc_counts_only_what_may_not_fit(sporder, n, deg, N, most):
+    """The long rows of an input that cannot outgrow the static scratch are not
+    counted, which would be a kernel, a readback and a synchronize."""
+    print(f"[spmm_launches] noalloc n={n} N={N}", flush=True)
+    p, i, v, B, out = case(n, deg, N)
+    names = kernels(lambda: sporder.spmm_csr_noalloc(p, i, v, B, out=out))
+    assert len(names) <= most and not any("count_long" in k for k in names)
