@@ -1085,11 +1085,16 @@ void launch_merge_g(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr,
                     const int32_t *ind, const float *val, int32_t N, const float *B, float *C) {
   constexpr int gpw = kWave / G; // row groups per wave
   // Span: about two groups per resident group slot, at least G * kSpmmDepth
-  // nonzeros (one full gather pipeline per group).
+  // nonzeros (one full gather pipeline per group).  Ragged widths below 2^20
+  // nonzeros: at least 64, or too few groups walk too many rows each (700,000
+  // nonzeros in 70,000 rows, N = 150: 177 us with 512, 124 with 64; 2 M: 248
+  // and 270).
   const int64_t groups = static_cast<int64_t>(ctx.num_cus) *
                          (ctx.max_threads_per_cu / kWave) * gpw * 2;
   int64_t span64 = ceil_div64(nnz > 0 ? nnz : 1, groups);
-  if (span64 < G * kSpmmDepth) span64 = G * kSpmmDepth;
+  int32_t least = G * kSpmmDepth;
+  if (least > 64 && nnz < (1 << 20) && is_ragged(N, B, C)) least = 64;
+  if (span64 < least) span64 = least;
   const int32_t span = static_cast<int32_t>(span64);
   const int64_t spans = ceil_div64(nnz, span);
   ctx.reserve(ws_bytes<int32_t>(static_cast<size_t>(spans) + 1));
@@ -1112,8 +1117,15 @@ void launch_merge_g(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr,
 void spmm_merge(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr,
                 const int32_t *ind, const float *val, int32_t N, const float *B,
                 float *C) {
-  if (N >= 4) {
-    const int32_t q = (N + 3) / 4; // float4 column slices
+  // Ragged widths take the row groups from 2^18 nonzeros on: 20,000 rows of 10,
+  // N = 101: 77 us a wave per span, 99 in row groups; power-law rows, 220,000
+  // nonzeros, N = 7 47 and 64; 40,000 rows of 10, N = 101 122 and 70.  Up to 8
+  // columns have 8 lanes to load the nonzeros (power-law rows, 600,000 of 12,
+  // N = 7: 978 -> 421 us, 667 a wave per span).
+  const bool ragged = is_ragged(N, B, C);
+  if (N >= 4 && !(ragged && nnz <= (1 << 18))) {
+    int32_t q = (N + 3) / 4; // float4 column slices
+    if (ragged && q <= 2) q = 8;
     if (q <= 1) {
       launch_merge_g<1>(ctx, n, nnz, ptr, ind, val, N, B, C);
     } else if (q <= 2) {
@@ -1131,7 +1143,7 @@ void spmm_merge(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr,
     }
     return;
   }
-  // Widths below 4: one wave per span, lanes over columns.
+  // One wave per span, lanes over columns.
   int64_t slots = static_cast<int64_t>(ctx.num_cus) * (ctx.max_threads_per_cu / kWave) * 2;
   int64_t span64 = ceil_div64(nnz > 0 ? nnz : 1, slots);
   if (span64 < 32) span64 = 32;

@@ -60,3 +60,16 @@ def test_noalloc_counts_only_what_may_not_fit(sporder, n, deg, N, most):
     p, i, v, B, out = case(n, deg, N)
     names = kernels(lambda: sporder.spmm_csr_noalloc(p, i, v, B, out=out))
     assert len(names) <= most and not any("count_long" in k for k in names)
+
+
+@pytest.mark.parametrize("N", [5, 47, 101])
+@pytest.mark.parametrize("n,deg,kernel", [(2_000, 8, "spmm_merge_path"),
+                                          (40_000, 8, "spmm_merge_v4")])
+def test_merge_spans_of_ragged_widths(sporder, n, deg, kernel, N):
+    """A wave per span up to 2^18 nonzeros, row groups (8 lanes or more) past
+    that: a few long walks in row groups took up to three times as long."""
+    print(f"[spmm_launches] merge n={n} N={N}", flush=True)
+    p, i, v, B, out = case(n, deg, N)
+    names = kernels(lambda: sporder.spmm_csr(p, i, v, B, out=out, algo="merge_path"))
+    assert any(kernel in k for k in names)
+    assert not any(f"spmm_merge_v4<{g}," in k for k in names for g in (1, 2, 4))
