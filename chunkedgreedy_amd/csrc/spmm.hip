@@ -590,9 +590,7 @@ __global__ void __launch_bounds__(kSpmmBlock)
     spmm_rowsplit_scalar(int32_t n, const int32_t *__restrict__ ptr,
                          const int32_t *__restrict__ ind,
                          const float *__restrict__ val, int32_t N,
-                         const float *__restrict__ B, float *__restrict__ C,
-                         const float *__restrict__ rs = nullptr,
-                         const float *__restrict__ cs = nullptr) {
+                         const float *__restrict__ B, float *__restrict__ C) {
   const int lane = lane_id();
   const int64_t wave0 =
       (blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x) / kWave;
@@ -606,12 +604,11 @@ __global__ void __launch_bounds__(kSpmmBlock)
         const int32_t q1 = q0 + seg < e ? q0 + seg : e;
         float acc = 0.0f;
         for (int32_t p = q0; p < q1; ++p) {
-          const float b = B[static_cast<int64_t>(ind[p]) * N + j];
-          acc = fmaf(val[p], cs != nullptr ? cs[p] * b : b, acc);
+          acc = fmaf(val[p], B[static_cast<int64_t>(ind[p]) * N + j], acc);
         }
         sum = (q0 == s) ? acc : sum + acc;
       }
-      C[row * N + j] = rs != nullptr ? rs[row] * sum : sum;
+      C[row * N + j] = sum;
     }
   }
 }

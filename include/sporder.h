@@ -405,7 +405,9 @@ SPORDER_API void sporder_hbm_stream(sporder_context_t ctx, int32_t op, int32_t n
  * processes on one GPU each use their own process's array.
  * Returns 0 when C is written, or SPORDER_SPMM_NOALLOC_TOO_LARGE (nothing
  * computed) when the input's long rows need more scratch than the array
- * holds.  Invalid arguments abort, as elsewhere.  Synchronous.
+ * holds, `cols` is a multiple of 4 and d_b and d_c are 16-byte aligned; at
+ * other widths and alignments such an input is computed by a slower kernel
+ * that needs no scratch.  Invalid arguments abort, as elsewhere.  Synchronous.
  */
 #define SPORDER_SPMM_NOALLOC_SCRATCH_BYTES (64u << 20)
 #define SPORDER_SPMM_NOALLOC_TOO_LARGE 1

@@ -1,7 +1,8 @@
 """sporder_spmm_csr_noalloc through the C ABI: equal bit for bit to
 sporder_spmm_csr (row-split), on two calls in a row with the second input
 smaller than the first (the static scratch keeps the first call's contents),
-on a width that takes the scalar kernel, and the size rejection."""
+on widths that need no scratch, and inputs whose long rows need more of it than
+there is: refused at whole, aligned widths, computed at the others."""
 
 import numpy as np
 import pytest
@@ -74,26 +75,30 @@ def test_noalloc_matches_row_split_twice(sporder, ctx):
     check_case(sporder, ctx, *small, N=64, seed=2)
 
 
-def test_noalloc_no_long_rows_and_scalar_width(sporder, ctx):
-    """No long rows at N = 32 (no segments), and N = 30 (the scalar kernel)."""
+def test_noalloc_no_long_rows_and_ragged_width(sporder, ctx):
+    """No long rows at N = 32 (no segments), and N = 30 (one launch)."""
     print("[noalloc] plain rows N=32, N=30", flush=True)
     plain = hub_csr(5000, 12, {}, 63)
     check_case(sporder, ctx, *plain, N=32, seed=3)
     check_case(sporder, ctx, *plain, N=30, seed=4)
 
 
-def test_noalloc_rejects_oversized_scratch(sporder, ctx):
-    """2048 rows of 1100 nonzeros at N = 4096: 6144 segment partial rows of
-    16 KiB need 96 MiB, more than the 64 MiB array: ValueError, C untouched;
-    a following call of normal size still matches."""
-    print("[noalloc] oversized rejection", flush=True)
+@pytest.fixture(scope="module")
+def oversized():
+    """2048 rows of 1100 nonzeros: at N = 4096, 6144 segment partial rows of
+    16 KiB need 96 MiB, more than the 64 MiB array."""
     n = 2048
     rng = np.random.default_rng(64)
-    ind_h = np.sort(np.stack([rng.choice(n, 1100, replace=False) for _ in range(n)]),
-                    axis=1).reshape(-1).astype(np.int32)
-    ptr_h = (np.arange(n + 1) * 1100).astype(np.int32)
-    val_h = rng.uniform(-1, 1, ind_h.size).astype(np.float32)
-    ptr, ind, val = to_dev(ptr_h, ind_h, val_h)
+    ind = np.sort(np.stack([rng.choice(n, 1100, replace=False) for _ in range(n)]), axis=1)
+    return ((np.arange(n + 1) * 1100).astype(np.int32), ind.reshape(-1).astype(np.int32),
+            rng.uniform(-1, 1, ind.size).astype(np.float32))
+
+
+def test_noalloc_rejects_oversized_scratch(sporder, ctx, oversized):
+    """ValueError, C untouched; a following call of normal size still matches."""
+    print("[noalloc] oversized rejection", flush=True)
+    n = 2048
+    ptr, ind, val = to_dev(*oversized)
     B = torch.ones((n, 4096), dtype=torch.float32, device="cuda:0")
     out = torch.zeros((n, 4096), dtype=torch.float32, device="cuda:0")
     with pytest.raises(ValueError, match="scratch"):
@@ -101,7 +106,24 @@ def test_noalloc_rejects_oversized_scratch(sporder, ctx):
     assert call_noalloc(sporder, ctx, ptr, ind, val, B, out) == _lib.SPMM_NOALLOC_TOO_LARGE
     assert int(torch.count_nonzero(out)) == 0
     del B, out
-    check_case(sporder, ctx, ptr_h, ind_h, val_h, N=128, seed=5)
+    check_case(sporder, ctx, *oversized, N=128, seed=5)
+
+
+def test_noalloc_computes_oversized_ragged(sporder, ctx, oversized):
+    """The same rows at N = 4095, and at N = 4096 on operands 4 bytes past a
+    16-byte boundary: computed without scratch, in the stated order."""
+    print("[noalloc] oversized, N = 4095", flush=True)
+    check_case(sporder, ctx, *oversized, N=4095, seed=7)
+    print("[noalloc] oversized, unaligned", flush=True)
+    n, N = 2048, 4096
+    ptr, ind, val = to_dev(*oversized)
+    gen = torch.Generator(device="cuda:0").manual_seed(8)
+    B, out = (torch.empty(n * N + 1, device="cuda:0")[1:].view(n, N) for _ in range(2))
+    B.copy_(torch.randn((n, N), generator=gen, device="cuda:0"))
+    ref, _ = sporder.spmm_csr(ptr, ind, val, B, algo="row_split", ctx=ctx)
+    out.fill_(float("nan"))
+    assert call_noalloc(sporder, ctx, ptr, ind, val, B, out) == 0
+    assert torch.equal(out.view(torch.int32), ref.view(torch.int32))
 
 
 def test_noalloc_leaves_device_memory_unchanged(sporder):
