@@ -530,7 +530,7 @@ template <int CELLS> struct WaveSketch {
   }
 
   // Up to this many live entries are merged rather than sorted (emit_lists).
-  static constexpr int kFewEntries = 12;
+  static constexpr int kFewEntries = 4;
 
   // select_top_k from the cells of logical lane L in physical lane L (< 32;
   // the upper half's values are not used).  NETWORK: past four cells, rows of
@@ -587,9 +587,10 @@ template <int CELLS> struct WaveSketch {
     }
     // Up to 128 live entries: one sorting network, about 700 wave instructions.
     // The merge below costs about 45 per emitted entry (k = 77 at CELLS = 10:
-    // some 3,500 a row, more than the row's counting), which is less for a few
-    // entries (csg of scrambled blocks of 600,000 rows, capacity 512: 446 ->
-    // 402 us).
+    // some 3,500 a row, more than the row's counting), one after another, which
+    // is less for hardly an entry (csg of scrambled blocks of 600,000 rows,
+    // capacity 512: 443 -> 402 us; merging up to 12, the 7-point stencil of
+    // 64,000 rows, capacity 256: 1.33 -> 1.45 ms).
     if constexpr (CELLS >= 3 && CELLS <= 4) {
       emit_sorted_lists(k, out, fk, fw);
       return;

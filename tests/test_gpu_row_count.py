@@ -115,13 +115,13 @@ CASES = {
     # chunks of 1024 rows past tier 1's nonzeros
     "groups90_long": lambda: groups(4500, 90, 24, 9),
     "groups127_long": lambda: groups(4500, 127, 36, 10),
-    # up to 12 entries are merged, up to 128 sorted (past four cells)
-    "groups12": lambda: groups(3100, 12, 21, 11),
-    "groups13": lambda: groups(3100, 13, 21, 12),
+    # up to 4 entries are merged, up to 128 sorted (past four cells)
+    "groups4": lambda: groups(3100, 4, 21, 11),
+    "groups5": lambda: groups(3100, 5, 21, 12),
     "groups128": lambda: groups(3100, 128, 21, 13),
     "groups129": lambda: groups(3100, 129, 21, 14),
-    "scattered12": lambda: groups(3100, 12, 21, 15, scatter=True),
-    "scattered13": lambda: groups(3100, 13, 21, 16, scatter=True),
+    "scattered4": lambda: groups(3100, 4, 21, 15, scatter=True),
+    "scattered5": lambda: groups(3100, 5, 21, 16, scatter=True),
     "scattered128": lambda: groups(3100, 128, 21, 17, scatter=True),
     "scattered129": lambda: groups(3100, 129, 21, 18, scatter=True),
 }
