@@ -132,8 +132,9 @@ __device__ __forceinline__ void register_sort_keys(uint32_t *keys, int32_t lo, i
 // Tier 1 is sized for two workgroups per CU, which needs 8 waves per SIMD and
 // so at most 64 VGPRs; the bound asks the compiler for that.  Capacities of
 // 256 slots and more (CELLS >= 8) would spill to scratch under it and keep
-// one workgroup per CU instead.  Tier 2 has 4 waves per SIMD; up to capacity 128 they are held to 5 waves'
-// registers (96), which leaves a SIMD room for two waves of the global path.
+// one workgroup per CU instead.  Tier 2 has 4 waves per SIMD; up to capacity
+// 128 they are held to 5 waves' registers (96), which leaves a SIMD room for
+// two waves of the global path.
 template <int CELLS, int KEYCAP>
 constexpr int local_eu_waves() {
   return KEYCAP <= 16384 ? (CELLS <= 7 ? 8 : 4) : (CELLS <= 4 ? 5 : 4);
@@ -146,7 +147,7 @@ constexpr int local_eu_waves() {
 constexpr int32_t kSerialItems = 14;
 
 // Entries of each wave's counting table (row_count.hpp): what the tier's LDS
-// leaves.  Tier 1: 120, with which two workgroups still share a CU (81,752 of
+// leaves.  Tier 1: 120, with which two workgroups still share a CU (81,760 of
 // 81,920 bytes each).  Tier 2 of chunks up to 1024 rows: 192, which leaves a CU
 // room for two workgroups of the global path at capacity 128.
 template <int KEYCAP, int ROWCAP> constexpr int local_table_entries() {
@@ -820,6 +821,7 @@ void launch_tier(Context &ctx, int32_t n, int32_t k, int32_t chunk_size, int32_t
   if (grid <= 0) return;
   using Lds = LocalLds<CELLS, KEYCAP, ROWCAP, 1 << NB_LOG2>;
   static_assert(sizeof(Lds) <= (KEYCAP <= 16384 ? 80 : 160) * 1024, "workgroups per CU");
+  static_assert(KEYCAP != kT1Keys || sizeof(Lds) == 81760, "local_table_entries states it");
   chunk_local_sketch_kernel<CELLS, KEYCAP, ROWCAP, NB_LOG2, CLAIM, COUNT>
       <<<dim3(static_cast<unsigned>(grid)), kLocalThreads, sizeof(Lds), ctx.stream>>>(
           n, k, chunk_size, lb, d_ptr, d_ind, d_table, list, list_count, ovf, ovf_count,
