@@ -963,9 +963,13 @@ int small_group(int32_t N) {
 // saves three of four (in us, against the other launches; 40,000 rows of 10):
 // N = 1 30 and 35, N = 30 36 and 39, N = 47 39 and 42; past 128 columns it has
 // few rows in a workgroup (N = 150: 73 and 69), and on larger matrices its long
-// rows keep to one CU (power-law, 100,000 rows, N = 30: 245 and 202).
-bool is_small(int32_t nnz, int32_t N, const float *B, const float *C) {
-  return is_ragged(N, B, C) && nnz <= (1 << (small_group(N) == 64 ? 18 : 19));
+// rows keep to one CU (power-law, 100,000 rows, N = 30: 245 and 202).  Many
+// rows of hardly a nonzero are not small either: past four times the lanes that
+// the device holds (1 M rows, 400,000 nonzeros, N = 1: 93 and 66; 300,000 rows,
+// N = 30: 51 and 62, N = 47: 72 and 65).
+bool is_small(int32_t n, int32_t nnz, int32_t N, const float *B, const float *C) {
+  const int group = small_group(N);
+  return is_ragged(N, B, C) && nnz <= (1 << (group == 64 ? 18 : 19)) && n <= (1 << 21) / group;
 }
 
 template <int G, int V, bool RG>
@@ -1025,7 +1029,7 @@ void spmm_rowsplit(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr,
                    const SpmmScale &sc = SpmmScale{}) {
   if (seg_cap < 0) seg_cap = max_segments(nnz);
   if (long_cap < 0) long_cap = max_long_rows(nnz);
-  if (tiles == nullptr && is_small(nnz, N, B, C) && w.ctl != nullptr) {
+  if (tiles == nullptr && is_small(n, nnz, N, B, C) && w.ctl != nullptr) {
     launch_small(ctx, n, ptr, ind, val, N, B, C, sc);
     return;
   }
@@ -1118,11 +1122,12 @@ void spmm_merge(Context &ctx, int32_t n, int32_t nnz, const int32_t *ptr,
   // N = 101: 77 us a wave per span, 99 in row groups; power-law rows, 220,000
   // nonzeros, N = 7 47 and 64; 40,000 rows of 10, N = 101 122 and 70.  Up to 8
   // columns have 8 lanes to load the nonzeros (power-law rows, 600,000 of 12,
-  // N = 7: 978 -> 421 us, 667 a wave per span).
+  // N = 7: 978 -> 421 us, 667 a wave per span) unless most rows have hardly one
+  // (1 M rows, 400,000 nonzeros: 113 us with two lanes, 178 with eight).
   const bool ragged = is_ragged(N, B, C);
   if (N >= 4 && !(ragged && nnz <= (1 << 18))) {
     int32_t q = (N + 3) / 4; // float4 column slices
-    if (ragged && q <= 2) q = 8;
+    if (ragged && q <= 2 && nnz / 4 >= n) q = 8;
     if (q <= 1) {
       launch_merge_g<1>(ctx, n, nnz, ptr, ind, val, N, B, C);
     } else if (q <= 2) {
@@ -1247,7 +1252,7 @@ int32_t sporder_spmm_csr_noalloc(sporder_context_t h, int32_t n, int32_t nnz,
   Context &ctx = h->impl;
   char *base = static_cast<char *>(noalloc_scratch(ctx.device));
   std::lock_guard<std::mutex> call_lock(noalloc_call_mu[ctx.device]);
-  if (is_small(nnz, cols, d_b, d_c)) { // no scratch
+  if (is_small(n, nnz, cols, d_b, d_c)) { // no scratch
     launch_small(ctx, n, d_ptr, d_ind, d_val, cols, d_b, d_c);
     ctx.sync();
     return 0;

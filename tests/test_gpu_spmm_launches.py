@@ -51,6 +51,15 @@ def test_small_calls_are_one_launch(sporder, how, N):
     assert len(names) == 1 and "spmm_rows_small" in names[0]
 
 
+@pytest.mark.parametrize("N", [1, 47])
+def test_many_empty_rows_are_not_small(sporder, N):
+    """400,000 rows of one nonzero."""
+    print(f"[spmm_launches] empty rows N={N}", flush=True)
+    p, i, v, B, out = case(400_000, 1, N)
+    names = kernels(lambda: sporder.spmm_csr(p, i, v, B, out=out))
+    assert not any("spmm_rows_small" in k for k in names)
+
+
 @pytest.mark.parametrize("n,deg,N,most", [(2_000, 8, 30, 1), (2_000, 8, 47, 1),
                                           (70_000, 10, 3, 4), (70_000, 10, 47, 4)])
 def test_noalloc_counts_only_what_may_not_fit(sporder, n, deg, N, most):
