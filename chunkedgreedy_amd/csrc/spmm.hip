@@ -25,12 +25,16 @@
 // launch (so one hub row does not serialise the whole SpMM), and a third
 // launch adds each long row's partials in the stated order.  For N <= 32
 // (8 or more rows per wave) the row groups of a wave claim its 64 rows
-// dynamically, so short rows do not wait for a long neighbour.
+// dynamically, so short rows do not wait for a long neighbour (ragged widths:
+// from kClaimedRows rows on).  Small calls of ragged widths do all of it in one
+// launch (spmm_rows_small).
 //
 // Merge-path: the nonzeros are cut into equal spans per wave (a row longer
 // than a span is split); each span's partial row sums are added into C with
 // atomics after the short rows are written directly.  The result equals the
-// row-split one up to the rounding of the split rows.
+// row-split one up to the rounding of the split rows.  Row groups take a span
+// each, as above; below 4 columns, and on small matrices at ragged widths, a
+// wave does.
 #include "common.hpp"
 #include "philox.hpp"
 
